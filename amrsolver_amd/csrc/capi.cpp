@@ -1080,18 +1080,6 @@ int get_tiles(amr_boxtab_s* bt, const FusedConfig& cfg, bool level, TileTable** 
   return AMR_OK;
 }
 
-FusedConfig default_config(const amr_boxtab_s* bt) {
-  // pick the largest tile that does not exceed the smallest box extent
-  int mnx = 1 << 30, mny = 1 << 30;
-  for (auto& B : bt->bt.h_boxes) {
-    mnx = std::min(mnx, B.hi[0] - B.lo[0] + 1);
-    mny = std::min(mny, B.hi[1] - B.lo[1] + 1);
-  }
-  FusedConfig c{16, 16, 64};
-  if (mnx < 16 || mny < 16) c = FusedConfig{8, 8, 64};
-  return c;
-}
-
 // The fused kernel takes any box (tiles overhanging a box in x or y are
 // masked); it skips only shapes whose tiles would be mostly idle.
 bool fused_fits(const amr_boxtab_s* bt, const FusedConfig& cfg, bool level = false) {
@@ -1105,20 +1093,76 @@ bool fused_fits(const amr_boxtab_s* bt, const FusedConfig& cfg, bool level = fal
   return 2 * cells_ >= lanes;
 }
 
+// Tiles per box of a tiling, and its estimated time: a tile costs a plane
+// iteration per plane plus three for the pipeline; `slots` workgroups fit the
+// chip at once (the 16x16 kernels two per CU, KEEP6 one, 8x8 columns eight),
+// and an iteration takes 1.35 times as long once the CUs are shared (128x64x64
+// viscous KEEP4, self-loading form: 64 tiles of 32 planes 3.6 us an
+// iteration, 512 tiles of 4 planes 5.0 us).
+int64_t tile_count(const amr_boxtab_s* bt, const FusedConfig& cfg, int64_t* iters = nullptr, int* longest = nullptr) {
+  int64_t n = 0, it = 0;
+  int mx = 0;
+  for (auto& B : bt->bt.h_boxes) {
+    const int64_t cols = int64_t((B.hi[0] - B.lo[0] + cfg.tx) / cfg.tx) * ((B.hi[1] - B.lo[1] + cfg.ty) / cfg.ty);
+    const int nz = B.hi[2] - B.lo[2] + 1, full = nz / cfg.tz, rem = nz % cfg.tz;
+    n += cols * (full + (rem ? 1 : 0));
+    it += cols * (int64_t(full) * (cfg.tz + 3) + (rem ? rem + 3 : 0));
+    mx = std::max(mx, std::min(nz, cfg.tz) + 3);
+  }
+  if (iters) *iters = it;
+  if (longest) *longest = mx;
+  return n;
+}
+
+double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedConfig& cfg) {
+  int64_t it = 0;
+  int mx = 0;
+  const int64_t n = tile_count(bt, cfg, &it, &mx);
+  const int64_t slots = 256 * (cfg.tx * cfg.ty == 64 ? 8 : (sch.order_keep == 6 ? 1 : 2));
+  if (n <= std::max<int64_t>(256, slots / 2)) return mx;
+  // whole rounds of the longest tiles while there are few, an even load later
+  const double rounds = n <= 4 * slots ? double((n + slots - 1) / slots) * mx : double(it) / slots;
+  return 1.35 * std::max(rounds, double(mx));
+}
+
+// The tiling of a table that has not been autotuned: 16x16 columns (in the
+// self-loading form where there is one) unless they would be mostly idle,
+// with the plane count of least estimated time -- short tiles where a level
+// has too few columns to fill the chip (32x24x20 in 8 boxes: 8x8x64 took
+// 90 us a right-hand side, 16x16x4 takes 30).
+FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
+  FusedConfig c{16, 16, 64};
+  if (fused_self_supported(sch, 16, 16)) c.form = 1;
+  if (!fused_fits(bt, c)) c = FusedConfig{8, 8, 64};
+  double best = 0.0;
+  FusedConfig out = c;
+  for (int tz : {64, 32, 16, 8, 4}) {
+    c.tz = tz;
+    const double t = tiling_time(bt, sch, c);
+    if (tz == 64 || t < best) {
+      best = t;
+      out = c;
+    }
+  }
+  return out;
+}
+
 FusedConfig choose_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
   const std::string key = scheme_key(sch);
   auto tk = bt->ctx->tuned.find(key);
   if (tk != bt->ctx->tuned.end()) return tk->second;
   auto tb = bt->tuned.find(key);
   if (tb != bt->tuned.end()) return tb->second;
-  return default_config(bt);
+  return default_config(bt, sch);
 }
 
 // Whether the fused stage kernel handles this scheme on this table.
 bool fused_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, FusedConfig* out, bool level = false) {
   FusedConfig cfg = choose_config(bt, sch);
   if (out) *out = cfg;
-  if (bt->walls) return false;  // the wall flux corrections run in the pass-structured kernels
+  // fluxes next to walls: the self-loading form (WallRows), else the
+  // pass-structured kernels' corrections
+  if (bt->wall_args.nkeep_blk > 0 && cfg.form != 1) return false;
   if (sch.rhs_source && bt->usrc_fn) return false;  // the user's source runs between assembly and combination
   return cfg.tx > 0 && fused_supported(sch, cfg.tx, cfg.ty) && fused_fits(bt, cfg, level);
 }
@@ -1446,6 +1490,7 @@ Cover kernel_cover(const amr_boxtab_s* bt, bool level) {
 // reads periodic images through box tiles).
 bool level_possible(amr_boxtab_s* bt, const amr_scheme_t& sch, DescSet* ds1, DescSet* dsin, DescSet* dout) {
   if (!bt->cover.on || wrap_ok(bt, dsin)) return false;
+  if (bt->wall_args.nkeep_blk > 0) return false;  // the rows next to a wall are found box by box
   if (!level_ok(bt, dsin) || !level_ok(bt, dout) || (ds1 && !level_ok(bt, ds1))) return false;
   if (sch.rhs_source && !(bt->src && level_ok(bt, bt->src.get()))) return false;
   return true;
@@ -1491,7 +1536,7 @@ void desc_layout(DescSet* ds) {
 // read the periodic images of its own cells, which costs less).
 bool nb_direct(amr_boxtab_s* bt, const amr_scheme_t& sch, bool level, DescSet* dsin) {
   desc_layout(dsin);
-  return !level && bt->nbmap.on && sch.order_keep <= 4 && dsin->span32 == 1 &&
+  return !level && bt->nbmap.on && bt->wall_args.nkeep_blk == 0 && sch.order_keep <= 4 && dsin->span32 == 1 &&
          fused_path(bt, sch, nullptr, level) && !wrap_ok(bt, dsin);
 }
 
@@ -1586,8 +1631,11 @@ int do_stage(amr_boxtab_s* bt, const amr_closures_t& cls, const amr_scheme_t& sc
     const Cover cov = kernel_cover(bt, level);
     NbMap nbm = !uncov_u0 && nb_direct(bt, sch, level, dsin) ? bt->nbmap : NbMap{};
     nbm.ustride = nbm.on && dsin->ustride == 1 ? 1 : 0;
+    WallRows wr{};
+    if (bt->wall_args.nkeep_blk > 0)
+      wr = WallRows{1, bt->geom.lo_bc[1] == 6, bt->geom.hi_bc[1] == 6, bt->geom.dom_lo[1], bt->geom.dom_hi[1]};
     HIPCHK(launch_fused_stage(sch, cfg, wa, cov, us, tt->d, tt->n, bt->bt.d_boxes, c, sa, s1, dsin->d, dout->d,
-                              st, nbm));
+                              st, nbm, wr));
     return AMR_OK;
   }
   if (uncov_u0) return fail(AMR_ERR_ARG, "internal: uncovered ghost cells from U^n requested off the fused path");
@@ -1684,7 +1732,7 @@ int stage_coeffs(int order_rk, int stages_rk, double dt, int stage, int* nst, St
 // workspaces have equal strides.
 int uncovered_from_un(amr_boxtab_s* bt, const amr_scheme_t& sch, DescSet* dst, DescSet* const dw[2], bool* ok) {
   *ok = false;
-  if (!bt->srcmap.on || wrap_ok(bt, dst)) return AMR_OK;
+  if (!bt->srcmap.on || wrap_ok(bt, dst) || bt->wall_args.nkeep_blk > 0) return AMR_OK;
   const bool level = use_level_tiles(bt, sch, dst, dst, dw[0]);
   if (level && !level_ok(bt, dw[1])) return AMR_OK;
   // stages that read the other boxes' cells directly read uncovered ghost
@@ -1784,7 +1832,8 @@ int prepare_step_tables(amr_boxtab_s* bt, const amr_scheme_t& sch, const amr_fab
     if (narrow && (rc = build_fill_narrow(bt, dw))) return rc;
   }
   FusedConfig cfg = choose_config(bt, sch);
-  const bool fused = cfg.tx > 0 && fused_supported(sch, cfg.tx, cfg.ty) && !bt->walls;
+  const bool fused = cfg.tx > 0 && fused_supported(sch, cfg.tx, cfg.ty) &&
+                     (bt->wall_args.nkeep_blk == 0 || cfg.form == 1) && !(sch.rhs_source && bt->usrc_fn);
   TileTable* tt = nullptr;
   if (fused && fused_fits(bt, cfg) && (rc = get_tiles(bt, cfg, false, &tt))) return rc;
   if (fused && bt->cover.on && (rc = get_tiles(bt, cfg, true, &tt))) return rc;
@@ -3293,20 +3342,27 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
   for (auto& B : bt->bt.h_boxes) maxz = std::max(maxz, B.hi[2] - B.lo[2] + 1);
   const int maxz_level = level ? bt->cover.hi[2] - bt->cover.lo[2] + 1 : 0;  // level tiles run across boxes
   std::vector<FusedConfig> cand;
+  const bool self16 = fused_self_supported(*sch, 16, 16) && fused_fits(bt, FusedConfig{16, 16, 16});
   const int shapes[3][2] = {{16, 16}, {32, 8}, {8, 8}};
-  const int tzs[6] = {16, 24, 32, 48, 64, 128};
+  const int tzs[8] = {4, 8, 16, 24, 32, 48, 64, 128};
   for (int box_tiles = level ? 0 : 1; box_tiles <= 1; ++box_tiles)
     for (auto& sh : shapes)
       for (int tz : tzs) {
         FusedConfig c{sh[0], sh[1], tz, box_tiles};
         if (tz > 2 * (box_tiles ? maxz : maxz_level) && tz != 16) continue;
+        // short tiles only where longer ones leave the chip idle
+        if (tz < 16 && tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz}) >= 1024) continue;
         if (!(fused_supported(*sch, c.tx, c.ty) && fused_fits(bt, c, !box_tiles))) continue;
-        cand.push_back(c);
-        // the self-loading form of the same tiling
-        if (fused_self_supported(*sch, c.tx, c.ty)) {
-          c.form = 1;
-          cand.push_back(c);
+        // the self-loading form where there is one (TGV 256^3, KEEP4: 0.68
+        // ms a stage against 0.77; KEEP2 0.59 against 0.64), which also
+        // leaves 32x8 columns behind (1.2 ms); next to walls only that form
+        if (self16) {
+          if (!fused_self_supported(*sch, c.tx, c.ty) && (c.tx != 8 || bt->wall_args.nkeep_blk > 0)) continue;
+          c.form = c.tx == 16 ? 1 : 0;
+        } else if (bt->wall_args.nkeep_blk > 0) {
+          continue;
         }
+        cand.push_back(c);
       }
   if (cand.empty()) {
     bt->tuned[key] = FusedConfig{-1, 0, 0};

@@ -57,36 +57,7 @@ struct Cfg {
   static constexpr int NOUT = NREG - NT - NRING;
 };
 
-// LDS cell of a thread's second load slot in the self-loading form (16x16
-// viscous tiles): the ring threads load their ring cell, threads 64 ..
-// 64 + NOUT - 1 (waves 1 and 2) the other halo cells (rows 0 and RY-1,
-// columns 0 and RX-1, then the ring's four corners); -1 for threads with no
-// second cell
-template <class C, int TX>
-__device__ __forceinline__ int self_halo_cell(int tid, int ring_idx) {
-  constexpr int RX = C::RX, RY = C::RY;
-  constexpr int OB = 64;  // first thread of the other halo cells
-  static_assert(C::EARLY && C::RB + C::NRING == C::NT && OB + C::NOUT <= C::RB,
-                "self-loading layout needs the ring on the last wave");
-  if (tid >= C::RB) return ring_idx;
-  if (tid < OB || tid >= OB + C::NOUT) return -1;
-  const int o = tid - OB;
-  int i, j;
-  if (o < RX) { i = o; j = 0; }
-  else if (o < 2 * RX) { i = o - RX; j = RY - 1; }
-  else if (o < 2 * RX + RY - 2) { i = 0; j = o - 2 * RX + 1; }
-  else if (o < 2 * RX + 2 * (RY - 2)) { i = RX - 1; j = o - 2 * RX - (RY - 2) + 1; }
-  else {
-    const int q = o - 2 * RX - 2 * (RY - 2);
-    i = (q & 1) ? RX - 2 : 1;
-    j = (q & 2) ? RY - 2 : 1;
-  }
-  return j * RX + i;
-}
-
-// SELF: the self-loading form (every cell a thread reads from the plane
-// above its own is one it stored, so storing that plane needs no barrier;
-// 16x16 viscous tiles).  SRC: the stage may carry a user_source array or
+// SRC: the stage may carry a user_source array or
 // a body force (the code for them is compiled out otherwise).  NB: tiles
 // per box read every halo cell that another box of the level holds (its
 // periodic image included) from that box's array, through an owner map of
@@ -101,7 +72,7 @@ __device__ __forceinline__ int self_halo_cell(int tid, int ring_idx) {
 // halving the occupancy.  Order 6 holds more (six pairs per x/y face, two
 // more z carries): one wave per SIMD with up to 512 registers rather than
 // spills to scratch memory.
-template <int H, bool VISC, int TX, int TY, bool UCS, bool SELF, bool SRC, int NB>
+template <int H, bool VISC, int TX, int TY, bool UCS, bool SRC, int NB>
 __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H == 3 ? 1 : 2))) k_fused(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes,
                                                      Closures c, double co0, double co1, double co2, StageArgs sa,
                                                      WrapArgs wa, Cover cov, UncovSrc us, NbMap nbm,
@@ -110,17 +81,12 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
   using C = Cfg<H, VISC, TX, TY>;
   static_assert(!NB || (!UCS && H <= 2), "neighbour reads take tiles per box of KEEP order 2 or 4");
   constexpr int RX = C::RX, HX = C::HX, PL = C::PL, NT = C::NT;
-  static_assert(!SELF || (VISC && TX == 16 && TY == 16 && C::NLOAD == 2 && C::EARLY),
-                "the self-loading form takes 16x16 viscous tiles");
   __shared__ double s_q[2][NPRIM * PL];
   __shared__ double s_px[VISC ? 4 : 1][TY][TX + 2];
   __shared__ double s_py[VISC ? 4 : 1][TY + 2][TX];
   __shared__ double s_fx[5][TY][TX + 1];
   __shared__ double s_fy[5][TY + 1][TX];
   __shared__ unsigned s_um[UCS ? C::NLOAD * NT : 1];
-  // KEEP part of the extra faces, across barrier (c) (self-loading form:
-  // s_fx/s_fy column TX / row TY may still be read for the plane below)
-  __shared__ double s_fe[SELF ? 5 : 1][SELF ? TX + TY : 1];
 
   const TileDev T = tiles[blockIdx.x];
   if (T.nz <= 0 || !box_active(sa, T.box)) return;  // uniform: the whole workgroup leaves
@@ -168,17 +134,9 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
     ring_idx = (ring_b + HX) * RX + (ring_a + HX);
   }
 
-  // LDS cell of each load slot (-1: loaded, not stored).  First form: slot
-  // s holds cell tid + s*NT.  Self-loading form: slot 0 is the own cell,
-  // slot 1 the cell self_halo_cell gives.
-  int scell[C::NLOAD];
-#pragma unroll
-  for (int s = 0; s < C::NLOAD; ++s) {
-    if constexpr (SELF) scell[s] = s == 0 ? own : self_halo_cell<C, TX>(tid, ring_idx);
-    else scell[s] = tid + s * NT < C::NREG ? tid + s * NT : -1;
-  }
-  // cell a slot loads: lanes with nothing to store load a region cell
-  auto load_cell = [&](int s) { return scell[s] >= 0 ? scell[s] : (SELF ? own : C::NREG - 1); };
+  // load slot s holds LDS cell tid + s*NT; lanes with nothing to store load
+  // the region's last cell
+  auto load_cell = [&](int s) { return min(tid + s * NT, C::NREG - 1); };
 
   // per-lane element offsets of the loaded plane cells; plane bases are
   // wave-uniform
@@ -333,8 +291,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
     double* sq = s_q[p & 1];
 #pragma unroll
     for (int s = 0; s < C::NLOAD; ++s) {
-      const int cell = SELF ? scell[s] : tid + s * NT;
-      if (SELF ? cell >= 0 : cell < C::NREG) {
+      const int cell = tid + s * NT;
+      if (cell < C::NREG) {
         double q[6];
         cons2prim(pre[s][0], pre[s][1], pre[s][2], pre[s][3], pre[s][4], c, q);
 #pragma unroll
@@ -406,10 +364,7 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
     if (VISC && ring_kind >= 0)
 #pragma unroll
       for (int n = 0; n < 4; ++n) rs[n] = sq[(QU + n) * PL + ring_idx];
-    // (b) plane c+1 visible.  The self-loading form reads plane c+1 only at
-    // cells the thread stored itself; it keeps the barrier while loading the
-    // planes below the tile, whose iterations have no other one
-    if (!SELF || cpl <= k0 - 1) __syncthreads();
+    __syncthreads();  // (b) plane c+1 visible
     if (cpl < k0 - 1 || (!VISC && H == 1 && cpl < k0)) {  // uniform: only loading planes below the tile
       if (H == 3 && cpl == k0 - 2) {
         // (k0, k0-3): the first face's (c, c-3) pair
@@ -520,10 +475,7 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
         double* dst = isx ? &s_fx[0][e][TX] : &s_fy[0][TY][e];
         const int cs = isx ? TY * (TX + 1) : (TY + 1) * TX;
 #pragma unroll
-        for (int n = 0; n < 5; ++n) {
-          if (SELF) s_fe[n][tid] = f[n];
-          else dst[n * cs] = f[n];
-        }
+        for (int n = 0; n < 5; ++n) dst[n * cs] = f[n];
       }
       // (c) viscous x/y fluxes visible; below the tile this barrier instead
       // keeps the next store from overwriting the plane just read
@@ -561,7 +513,7 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
           const double* pv = isx ? &s_px[0][e][TX] : &s_py[0][TY][e];
           const int pcs = isx ? TY * (TX + 2) : (TY + 2) * TX, pst = isx ? 1 : TX;
 #pragma unroll
-          for (int n = 0; n < 5; ++n) f[n] = SELF ? s_fe[n][q] : dst[n * cs];
+          for (int n = 0; n < 5; ++n) f[n] = dst[n * cs];
           f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
           for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (pv[n * pcs] + pv[n * pcs + pst]);
@@ -671,11 +623,11 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
   }
 }
 
-#define AMR_FUSED_LAUNCH(UCS_, SELF_, SRC_, NB_)                                                              \
-  hipLaunchKernelGGL((k_fused<H, VISC, TX, TY, UCS_, SELF_, SRC_, NB_>), dim3(ntiles), dim3(TX * TY), 0, st, tiles, \
+#define AMR_FUSED_LAUNCH(UCS_, SRC_, NB_)                                                                     \
+  hipLaunchKernelGGL((k_fused<H, VISC, TX, TY, UCS_, SRC_, NB_>), dim3(ntiles), dim3(TX * TY), 0, st, tiles, \
                      boxes, c, co[0], co[1], co[2], sa, wa, cov, us, nbm, s1, sin, out)
 
-template <int H, bool VISC, int TX, int TY, bool SELF>
+template <int H, bool VISC, int TX, int TY>
 void launch_t(const TileDev* tiles, int ntiles, const BoxDev* boxes, const Closures& c, const double co[3],
               const StageArgs& sa, const WrapArgs& wa, const Cover& cov, const UncovSrc& us, const NbMap& nbm,
               const Fab* s1, const Fab* sin, const Fab* out, hipStream_t st) {
@@ -683,21 +635,21 @@ void launch_t(const TileDev* tiles, int ntiles, const BoxDev* boxes, const Closu
   if constexpr (H <= 2) {
     if (nbm.on) {
       if (nbm.ustride) {
-        if (src) AMR_FUSED_LAUNCH(false, SELF, true, 2);
-        else AMR_FUSED_LAUNCH(false, SELF, false, 2);
+        if (src) AMR_FUSED_LAUNCH(false, true, 2);
+        else AMR_FUSED_LAUNCH(false, false, 2);
       } else {
-        if (src) AMR_FUSED_LAUNCH(false, SELF, true, 1);
-        else AMR_FUSED_LAUNCH(false, SELF, false, 1);
+        if (src) AMR_FUSED_LAUNCH(false, true, 1);
+        else AMR_FUSED_LAUNCH(false, false, 1);
       }
       return;
     }
   }
   if (us.on) {
-    if (src) AMR_FUSED_LAUNCH(true, SELF, true, 0);
-    else AMR_FUSED_LAUNCH(true, SELF, false, 0);
+    if (src) AMR_FUSED_LAUNCH(true, true, 0);
+    else AMR_FUSED_LAUNCH(true, false, 0);
   } else {
-    if (src) AMR_FUSED_LAUNCH(false, SELF, true, 0);
-    else AMR_FUSED_LAUNCH(false, SELF, false, 0);
+    if (src) AMR_FUSED_LAUNCH(false, true, 0);
+    else AMR_FUSED_LAUNCH(false, false, 0);
   }
 }
 #undef AMR_FUSED_LAUNCH
@@ -709,14 +661,14 @@ bool launch_shape(const amr_scheme_t& s, const TileDev* tiles, int ntiles, const
                   hipStream_t st) {
   const bool v = s.rhs_visc != 0;
   if (s.order_keep == 6) {
-    if (v) launch_t<3, true, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    else launch_t<3, false, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    if (v) launch_t<3, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    else launch_t<3, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   } else if (s.order_keep == 4) {
-    if (v) launch_t<2, true, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    else launch_t<2, false, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    if (v) launch_t<2, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    else launch_t<2, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   } else if (s.order_keep == 2) {
-    if (v) launch_t<1, true, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    else launch_t<1, false, TX, TY, false>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    if (v) launch_t<1, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    else launch_t<1, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   } else {
     return false;
   }
@@ -732,24 +684,17 @@ bool fused_supported(const amr_scheme_t& s, int tx, int ty) {
   return (tx == 16 && ty == 16) || (tx == 8 && ty == 8) || (tx == 32 && ty == 8);
 }
 
-bool fused_self_supported(const amr_scheme_t& s, int tx, int ty) {
-  return fused_supported(s, tx, ty) && s.order_keep <= 4 && s.rhs_visc && tx == 16 && ty == 16;
-}
-
 hipError_t launch_fused_stage(const amr_scheme_t& s, const FusedConfig& cfg, const WrapArgs& wa, const Cover& cov,
                               const UncovSrc& us, const TileDev* tiles, int ntiles, const BoxDev* boxes,
                               const Closures& c, const StageArgs& sa, const Fab* s1, const Fab* sin, const Fab* out,
-                              hipStream_t st, const NbMap& nbm) {
-  if (nbm.on && (us.on || s.order_keep > 4)) return hipErrorInvalidValue;
+                              hipStream_t st, const NbMap& nbm, const WallRows& wr) {
+  if (cfg.form == 1)
+    return launch_fused_self(s, cfg, wa, cov, us, tiles, ntiles, boxes, c, sa, s1, sin, out, st, nbm, wr);
+  if ((nbm.on && (us.on || s.order_keep > 4)) || wr.on) return hipErrorInvalidValue;
   double co[3];
   keep_coefficients(s.order_keep, co);
   bool ok = false;
-  if (cfg.form == 1) {
-    if (!fused_self_supported(s, cfg.tx, cfg.ty)) return hipErrorInvalidValue;
-    if (s.order_keep == 4) launch_t<2, true, 16, 16, true>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    else launch_t<1, true, 16, 16, true>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    ok = true;
-  } else if (cfg.tx == 16 && cfg.ty == 16)
+  if (cfg.tx == 16 && cfg.ty == 16)
     ok = launch_shape<16, 16>(s, tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   else if (cfg.tx == 8 && cfg.ty == 8)
     ok = launch_shape<8, 8>(s, tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);

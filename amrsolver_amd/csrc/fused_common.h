@@ -22,11 +22,9 @@ struct VDer {
 
 // ViscousFluxes (CNS_hydro_K.h:133-171), components UMX..UET (URHO is 0)
 template <bool WX, bool WY, bool WZ>
-__device__ __forceinline__ void visc_flux(const VDer& d, const Closures& c, double fx[4], double fy[4],
-                                          double fz[4]) {
+__device__ __forceinline__ void visc_flux_of(const VDer& d, double mu, double lambda, double fx[4], double fy[4],
+                                             double fz[4]) {
   double div = d.dudx + d.dvdy + d.dwdz;
-  double mu = visc(c, d.T);
-  double lambda = cond(c, d.T, mu);
   double r1_3 = 1.0 / 3.0;
   double tauxx = 2.0 * mu * (d.dudx - r1_3 * div);
   double tauxy = mu * (d.dudy + d.dvdx);
@@ -52,6 +50,13 @@ __device__ __forceinline__ void visc_flux(const VDer& d, const Closures& c, doub
     fz[2] = -tauzz;
     fz[3] = -lambda * d.dTdz - tauxz * d.ux - tauyz * d.uy - tauzz * d.uz;
   }
+}
+
+template <bool WX, bool WY, bool WZ>
+__device__ __forceinline__ void visc_flux(const VDer& d, const Closures& c, double fx[4], double fy[4],
+                                          double fz[4]) {
+  const double mu = visc(c, d.T);
+  visc_flux_of<WX, WY, WZ>(d, mu, cond(c, d.T, mu), fx, fy, fz);
 }
 
 // KEEP face flux in direction NRM at the face below LDS cell `idx`; cells

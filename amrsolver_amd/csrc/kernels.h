@@ -410,9 +410,18 @@ constexpr int UNCOV_MAX_ZBLK = 32;
 bool fused_supported(const amr_scheme_t& s, int tx, int ty);
 // the self-loading form of the fused kernel (FusedConfig::form 1) applies
 bool fused_self_supported(const amr_scheme_t& s, int tx, int ty);
+// bc 6 walls in y for the self-loading form: the domain's y bounds and which
+// of them are walls (tiles per box; box boundaries decide which tiles touch).
+struct WallRows {
+  int on, lo_wall, hi_wall, dlo, dhi;
+};
+hipError_t launch_fused_self(const amr_scheme_t& s, const FusedConfig& cfg, const WrapArgs& wa, const Cover& cov,
+                             const UncovSrc& us, const TileDev* tiles, int ntiles, const BoxDev* boxes,
+                             const Closures& c, const StageArgs& sa, const Fab* s1, const Fab* sin, const Fab* out,
+                             hipStream_t st, const NbMap& nbm, const WallRows& wr);
 hipError_t launch_fused_stage(const amr_scheme_t& s, const FusedConfig& cfg, const WrapArgs& wa, const Cover& cov,
                               const UncovSrc& us, const TileDev* tiles, int ntiles, const BoxDev* boxes,
                               const Closures& c, const StageArgs& sa, const Fab* s1, const Fab* sin, const Fab* out,
-                              hipStream_t st, const NbMap& nbm = NbMap{});
+                              hipStream_t st, const NbMap& nbm = NbMap{}, const WallRows& wr = WallRows{});
 
 }  // namespace amr

@@ -382,7 +382,8 @@ int amr_set_tiling(amr_ctx_t ctx, const amr_scheme_t* sch, int tx, int ty, int t
 /* As amr_set_tiling, choosing also the form of the fused kernel: 0 the
  * first, 1 the self-loading one (16x16 tiles of a viscous KEEP 2/4 scheme:
  * each thread converts the cells of the next plane it reads itself, which
- * saves one workgroup barrier per plane).  The forms give the same bits.
+ * saves one workgroup barrier per plane, and every KEEP pair is formed once;
+ * the only form that runs next to bc 6 walls).  The forms give the same bits.
  * No reference counterpart. */
 int amr_set_tiling_form(amr_ctx_t ctx, const amr_scheme_t* sch, int tx, int ty, int tz, int form);
 
@@ -407,9 +408,10 @@ int amr_set_box_tiling(amr_ctx_t ctx, const amr_scheme_t* sch, int tx, int ty, i
 int amr_step_plan(amr_boxtab_t bt, const amr_scheme_t* sch, const amr_fab_t* state, int32_t info[6]);
 
 /* Time a whole step (fills and stages, the last one written to a workspace)
- * on `state` (ghost-filled, ng >= 3) under every compiled tiling that fits
+ * on `state` (ghost-filled, ng >= 3) under the compiled tilings that fit
  * the level -- tiles per box and, where the state is one array over the
- * level, tiles over the union of the boxes -- and keep the fastest for this
+ * level, tiles over the union of the boxes; of 16x16 columns the self-loading
+ * form alone where the scheme has it -- and keep the fastest for this
  * scheme on this box table (it clears an explicit amr_set_tiling for the
  * scheme).  Writes the choice to tiling[3] (tx,ty,tz; tx = -1 when only the
  * pass-structured kernels apply).  Synchronous; leaves `state` unchanged. */
