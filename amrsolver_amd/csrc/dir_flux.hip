@@ -239,7 +239,7 @@ __device__ __forceinline__ void add_visc_face(const WenoBrick& W, const BoxDev& 
 }
 
 template <int D, int LAST>
-__global__ void __launch_bounds__(WNT) k_weno_dir(const WenoBrick* __restrict__ bricks, const BoxDev* __restrict__ boxes,
+__global__ void __launch_bounds__(WNT, 4) k_weno_dir(const WenoBrick* __restrict__ bricks, const BoxDev* __restrict__ boxes,
                                                   Closures c, StageArgs sa, const Fab* __restrict__ sinf,
                                                   const Fab* __restrict__ accf, const Fab* __restrict__ s1f,
                                                   const Fab* __restrict__ outf, const Fab* __restrict__ pvf,
@@ -336,24 +336,36 @@ __global__ void __launch_bounds__(WNT) k_weno_dir(const WenoBrick* __restrict__ 
     for (int o = 1; o < 6; ++o) me = dmax(me, sv[7][l0 + o * st]);
     return me;
   };
-  auto face_comp = [&](int l0, double me, int n) {
-    double df[6], Pf[6];
+  // (the halves of the split fluxes, exact, are taken of the wave speed, the
+  // normal velocity and the pressure instead of every split value)
+  auto face_split = [&](int l0, double me, int n, double df[6], double Pf[6]) {
+    const double hme = 0.5 * me;
 #pragma unroll
     for (int o = 0; o < 6; ++o) {
       const int l = l0 + o * st;
-      const double ud = sv[5][l];
+      const double hud = 0.5 * sv[5][l];
       double flux;
-      if (n == URHO) flux = sv[1 + D][l];
-      else if (n == UET) flux = (sv[4][l] + sv[6][l]) * ud;
-      else if (n == 1 + D) flux = sv[n][l] * ud + sv[6][l];
-      else flux = sv[n][l] * ud;
-      df[o] = me * sv[n][l];
+      if (n == URHO) flux = 0.5 * sv[1 + D][l];
+      else if (n == UET) flux = (sv[4][l] + sv[6][l]) * hud;
+      else if (n == 1 + D) flux = sv[n][l] * hud + 0.5 * sv[6][l];
+      else flux = sv[n][l] * hud;
+      df[o] = hme * sv[n][l];
       Pf[o] = flux;
     }
-    double flx = weno5js(0.5 * (Pf[0] + df[0]), 0.5 * (Pf[1] + df[1]), 0.5 * (Pf[2] + df[2]),
-                         0.5 * (Pf[3] + df[3]), 0.5 * (Pf[4] + df[4]));
-    flx += weno5js(0.5 * (Pf[5] - df[5]), 0.5 * (Pf[4] - df[4]), 0.5 * (Pf[3] - df[3]),
-                   0.5 * (Pf[2] - df[2]), 0.5 * (Pf[1] - df[1]));
+  };
+  auto face_comp = [&](int l0, double me, int n, bool& ok) {
+    double df[6], Pf[6];
+    face_split(l0, me, n, df, Pf);
+    double flx = weno5js_fast(Pf[0] + df[0], Pf[1] + df[1], Pf[2] + df[2], Pf[3] + df[3], Pf[4] + df[4], ok);
+    flx += weno5js_fast(Pf[5] - df[5], Pf[4] - df[4], Pf[3] - df[3], Pf[2] - df[2], Pf[1] - df[1], ok);
+    return flx;
+  };
+  // outside the fast form's range
+  auto face_comp_plain = [&](int l0, double me, int n) {
+    double df[6], Pf[6];
+    face_split(l0, me, n, df, Pf);
+    double flx = weno5js(Pf[0] + df[0], Pf[1] + df[1], Pf[2] + df[2], Pf[3] + df[3], Pf[4] + df[4]);
+    flx += weno5js(Pf[5] - df[5], Pf[4] - df[4], Pf[3] - df[3], Pf[2] - df[2], Pf[1] - df[1]);
     return flx;
   };
   double* sF = &sv[0][0];  // [5][NF]
@@ -371,7 +383,10 @@ __global__ void __launch_bounds__(WNT) k_weno_dir(const WenoBrick* __restrict__ 
         const int n = u / G::NF, f = u - n * G::NF;
         const int fx = f % G::FX, fb = f / G::FX;
         const int l0 = fb * G::LX + fx;
-        Fu[r] = face_comp(l0, face_me(l0), n);
+        const double me = face_me(l0);
+        bool ok = true;
+        Fu[r] = face_comp(l0, me, n, ok);
+        if (!ok) Fu[r] = face_comp_plain(l0, me, n);
       }
     }
     __syncthreads();  // every stencil read done: the faces reuse the cell slots
@@ -392,8 +407,17 @@ __global__ void __launch_bounds__(WNT) k_weno_dir(const WenoBrick* __restrict__ 
         const int fx = f % G::FX, fb = f / G::FX;
         const int l0 = fb * G::LX + fx;
         const double me = face_me(l0);
+        bool ok = true;
 #pragma unroll
-        for (int n = 0; n < 5; ++n) F[r][n] = face_comp(l0, me, n);
+        for (int n = 0; n < 5; ++n) {
+          F[r][n] = face_comp(l0, me, n, ok);
+          // one component at a time: interleaved, the five take 240 VGPRs,
+          // two waves per SIMD, and run 1.3x slower
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!ok)
+#pragma unroll
+          for (int n = 0; n < 5; ++n) F[r][n] = face_comp_plain(l0, me, n);
         if (pvf) add_visc_face<D, G::FX>(W, bx, pvf[W.box], f, F[r]);
       }
     }
