@@ -847,6 +847,40 @@ int copy_uncovered(amr_boxtab_s* bt, const DescSet* from, const DescSet* to, con
 
 enum { UW_PRIMS = 1, UW_VISC = 2, UW_WENO = 4, UW_SLOPE = 8, UW_JST = 16 };
 
+// Brick table of the tube stages: side tables (so every box spans its
+// periodic y and z extents) and boxes 4 x 4 cells across.  Split bricks while
+// they fill less than a few rounds of the chip (one workgroup a CU): above
+// that the long bricks' throughput wins.
+int build_tube(amr_boxtab_s* bt) {
+  if (!bt->d_xside) return AMR_OK;
+  int64_t short_bricks = 0;
+  for (auto& B : bt->bt.h_boxes) {
+    if (B.hi[1] - B.lo[1] != 3 || B.hi[2] - B.lo[2] != 3) return AMR_OK;
+    short_bricks += (B.hi[0] - B.lo[0] + TUBE_SPLIT_NX) / TUBE_SPLIT_NX;
+  }
+  TubeWork& w = bt->uw.tube;
+  w.split = short_bricks <= TUBE_SPLIT_MAX;
+  const int most = w.split ? TUBE_SPLIT_NX : TUBE_NX;
+  std::vector<TubeBrick> h;
+  for (int b = 0; b < bt->bt.nbox; ++b) {
+    const BoxDev& B = bt->bt.h_boxes[b];
+    const amr_geom_t& g = bt->geoms[b];
+    const int len = B.hi[0] - B.lo[0] + 1, pieces = (len + most - 1) / most;
+    const int wrap = g.periodic[0] && B.lo[0] == g.dom_lo[0] && B.hi[0] == g.dom_hi[0] ? len : 0;
+    int x = B.lo[0];
+    for (int p = 0; p < pieces; ++p) {
+      const int nx = len / pieces + (p < len % pieces ? 1 : 0);
+      h.push_back(TubeBrick{b, x, nx, wrap});
+      x += nx;
+    }
+  }
+  HIPCHK(hipMalloc(&w.d, sizeof(TubeBrick) * h.size()));
+  HIPCHK(hipMemcpy(w.d, h.data(), sizeof(TubeBrick) * h.size(), hipMemcpyHostToDevice));
+  bt->uw_tables.push_back(w.d);
+  w.n = int(h.size());
+  return AMR_OK;
+}
+
 int ensure_unfused(amr_boxtab_s* bt, const amr_scheme_t& s) {
   int need = UW_PRIMS;
   if (s.rhs_visc) need |= UW_VISC;
@@ -936,6 +970,7 @@ int ensure_unfused(amr_boxtab_s* bt, const amr_scheme_t& s) {
       bt->uw.weno.n[d] = n;
     }
     bt->uw.weno.xside = bt->d_xside;
+    if (int rc = build_tube(bt)) return rc;
   }
   bt->uw_kinds = need;
   return AMR_OK;

@@ -59,6 +59,21 @@ struct WenoWork {
   // have kind 1 or 2: the passes then read no ghost cell (no fill needed)
   const XSide* xside = nullptr;
 };
+// Tube stages (tube_flux.hip): brick = up to TUBE_NX (split: TUBE_SPLIT_NX)
+// cells along x from x0 of a box 4 x 4 cells across, periodic in y and z;
+// wrap > 0: the box spans a periodic x extent of that many cells.
+struct TubeBrick {
+  int box, x0, nx, wrap;
+};
+constexpr int TUBE_NX = 15, TUBE_SPLIT_NX = 3, TUBE_SPLIT_MAX = 512;
+struct TubeWork {
+  TubeBrick* d = nullptr;
+  int n = 0;
+  bool split = false;
+};
+// One inviscid WENO (flux_euler 2) or MUSCL (0) stage of every box.
+hipError_t launch_tube(int flux_euler, const TubeWork& tw, const BoxDev* boxes, const Closures& c, const StageArgs& sa,
+                       const Fab* sin, const Fab* s1, const Fab* out, const XSide* xs, hipStream_t st);
 int weno_brick_count(const BoxTable& bt, int d);
 void weno_bricks(const BoxTable& bt, int d, const int* wrap, WenoBrick* out);
 
@@ -66,6 +81,7 @@ void weno_bricks(const BoxTable& bt, int d, const int* wrap, WenoBrick* out);
 // nbox Fab each).
 struct UnfusedWork {
   WenoWork weno;            // brick tables of the directional flux passes
+  TubeWork tube;            // brick table of the tube stages (d null: not such a table)
   Fab* prims = nullptr;     // NPRIM comps on grow(bx,3)
   Fab* nf[3] = {};          // NCONS comps on [lo, hi+1]^3
   Fab* pv[3] = {};          // NCONS comps on grow(bx,1)   (viscous)
