@@ -487,17 +487,15 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
       double f[5];
       keep_face<H, 0, PL>(sq, own, 1, co, cv, f);
       if (VISC) {
-        f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (s_px[n][tj][ti] + s_px[n][tj][ti + 1]);
+        for (int n = 0; n < 4; ++n) f[n + 1] = __builtin_fma(0.5, s_px[n][tj][ti] + s_px[n][tj][ti + 1], f[n + 1]);
       }
 #pragma unroll
       for (int n = 0; n < 5; ++n) s_fx[n][tj][ti] = f[n];
       keep_face<H, 1, PL>(sq, own, RX, co, cv, f);
       if (VISC) {
-        f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (s_py[n][tj][ti] + s_py[n][tj + 1][ti]);
+        for (int n = 0; n < 4; ++n) f[n + 1] = __builtin_fma(0.5, s_py[n][tj][ti] + s_py[n][tj + 1][ti], f[n + 1]);
       }
 #pragma unroll
       for (int n = 0; n < 5; ++n) s_fy[n][tj][ti] = f[n];
@@ -514,9 +512,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
           const int pcs = isx ? TY * (TX + 2) : (TY + 2) * TX, pst = isx ? 1 : TX;
 #pragma unroll
           for (int n = 0; n < 5; ++n) f[n] = dst[n * cs];
-          f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-          for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (pv[n * pcs] + pv[n * pcs + pst]);
+          for (int n = 0; n < 4; ++n) f[n + 1] = __builtin_fma(0.5, pv[n * pcs] + pv[n * pcs + pst], f[n + 1]);
 #pragma unroll
           for (int n = 0; n < 5; ++n) dst[n * cs] = f[n];
         }
@@ -524,9 +521,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
         const int jj = tid - C::XB;
         keep_face<H, 0, PL>(sq, (jj + HX) * RX + (TX + HX), 1, co, cv, f);
         if (VISC) {
-          f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-          for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (s_px[n][jj][TX] + s_px[n][jj][TX + 1]);
+          for (int n = 0; n < 4; ++n) f[n + 1] = __builtin_fma(0.5, s_px[n][jj][TX] + s_px[n][jj][TX + 1], f[n + 1]);
         }
 #pragma unroll
         for (int n = 0; n < 5; ++n) s_fx[n][jj][TX] = f[n];
@@ -534,9 +530,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
         const int ii = tid - C::YB;
         keep_face<H, 1, PL>(sq, (TY + HX) * RX + (ii + HX), RX, co, cv, f);
         if (VISC) {
-          f[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-          for (int n = 0; n < 4; ++n) f[n + 1] += 0.5 * (s_py[n][TY][ii] + s_py[n][TY + 1][ii]);
+          for (int n = 0; n < 4; ++n) f[n + 1] = __builtin_fma(0.5, s_py[n][TY][ii] + s_py[n][TY + 1][ii], f[n + 1]);
         }
 #pragma unroll
         for (int n = 0; n < 5; ++n) s_fy[n][TY][ii] = f[n];
@@ -580,9 +575,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
         keep_accum(co[2], z3p, fz);
       }
       if (VISC) {
-        fz[0] += 0.5 * (0.0 + 0.0);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) fz[n + 1] += 0.5 * (pfz_prev[n] + pfz_cur[n]);
+        for (int n = 0; n < 4; ++n) fz[n + 1] = __builtin_fma(0.5, pfz_prev[n] + pfz_cur[n], fz[n + 1]);
       }
       if (fin && ((cword >> ((((cpl - 1 - cov.lo[2]) >> cov.sh) * cplane + ccol) & 31)) & 1u)) {
         gdouble* po = gptr(O.p) + O.idx(gi, gj, cpl - 1);

@@ -88,17 +88,15 @@ __device__ __forceinline__ void keep_terms_xy(bool isx, double rho1, double ux1,
                                               double uz2, double ie2, double p2, double t[5]) {
   const double un1 = isx ? ux1 : uy1;
   const double un2 = isx ? ux2 : uy2;
-  const double massflx = fgQuad(rho1, rho2, un1, un2);
-  const double ke = 0.5 * (ux1 * ux2 + uy1 * uy2 + uz1 * uz2);
+  const double massflx = 0.25 * (rho1 + rho2) * (un1 + un2);
+  const double hm = 0.5 * massflx;
   t[URHO] = massflx;
-  const double cx = fghCubic(rho1, rho2, un1, un2, ux1, ux2);
-  const double cy = fghCubic(rho1, rho2, un1, un2, uy1, uy2);
-  const double pd = fDiv(p1, p2);
-  const double cxp = cx + pd, cyp = cy + pd;
-  t[UMX] = isx ? cxp : cx;
-  t[UMY] = isx ? cy : cyp;
-  t[UMZ] = fghCubic(rho1, rho2, un1, un2, uz1, uz2);
-  t[UET] = massflx * ke + fghCubic(rho1, rho2, un1, un2, ie1, ie2) + fgDiv(p1, p2, un1, un2);
+  const double cx = hm * (ux1 + ux2), cy = hm * (uy1 + uy2);
+  const double ps = p1 + p2;
+  t[UMX] = isx ? __builtin_fma(0.5, ps, cx) : cx;
+  t[UMY] = isx ? cy : __builtin_fma(0.5, ps, cy);
+  t[UMZ] = hm * (uz1 + uz2);
+  t[UET] = __builtin_fma(0.5, p1 * un2 + p2 * un1, hm * (ux1 * ux2 + uy1 * uy2 + uz1 * uz2) + hm * (ie1 + ie2));
 }
 
 // keep_face with the direction chosen per lane (isx: x face, stride 1;

@@ -28,9 +28,9 @@
 //
 // Measured (MI355X, us a stage; first form and its earlier self-loading
 // variant with three and two barriers and 6 pairs per x/y face pair -> this):
-// TGV 256^3 KEEP4 766 -> 675, KEEP2 640 -> 592; 192x160x128 with one array
-// per box 216 -> 191; the channel 96x128x64 between bc 6 walls, fills
-// included, 222 (pass-structured kernels) -> 67.  What bounds it now: latency
+// TGV 256^3 KEEP4 766 -> 660, KEEP2 640 -> 586; 192x160x128 with one array
+// per box 216 -> 189; the channel 96x128x64 between bc 6 walls, fills
+// included, 222 (pass-structured kernels) -> 65.  What bounds it now: latency
 // at two waves per SIMD (243 VGPRs, 78 KB of LDS); the VALU is busy about
 // half of the time, the LDS a fifth.
 #include "kernels.h"
@@ -425,7 +425,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
       double fz[5], t[5];
       zterms(qs, qm1, cv, t);  // (c, c-1)
 #pragma unroll
-      for (int n = 0; n < 5; ++n) fz[n] = 0.0 + co0 * t[n];
+      for (int n = 0; n < 5; ++n) fz[n] = co0 * t[n];
       if (H == 2) {
         // (c, c-2) is the previous plane's (c+1, c-1), carried in registers
         keep_accum(co1, zcarry, fz);
@@ -433,7 +433,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
         keep_accum(co1, zcarry, fz);
       }
 #pragma unroll
-      for (int n = 0; n < 4; ++n) fz[n + 1] += 0.5 * (pfz_prev[n] + pfz_cur[n]);
+      for (int n = 0; n < 4; ++n) fz[n + 1] = __builtin_fma(0.5, pfz_prev[n] + pfz_cur[n], fz[n + 1]);
       if (cpl > k0) {
         // the plane below is complete
         const int kp = cpl - 1;
@@ -494,7 +494,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
         const Cell e = lds_cell(s_q, own + 1), w = lds_cell(s_q, own - 1);
         pair_terms<0>(o, w, cv, t);
 #pragma unroll
-        for (int n = 0; n < 5; ++n) fx[n] = 0.0 + co0 * t[n];
+        for (int n = 0; n < 5; ++n) fx[n] = co0 * t[n];
         if (ti == 0)
 #pragma unroll
           for (int n = 0; n < 5; ++n) s_a[n][TX + TY + tj] = fx[n];
@@ -514,13 +514,13 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
 #pragma unroll
           for (int n = 0; n < 4; ++n) s_e[NP + n][xp] = vx[n];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) fx[n + 1] += 0.5 * (dpp_row<ROW_SHR1>(0.0, vx[n]) + vx[n]);
+        for (int n = 0; n < 4; ++n) fx[n + 1] = __builtin_fma(0.5, dpp_row<ROW_SHR1>(0.0, vx[n]) + vx[n], fx[n + 1]);
       }
       {
         const Cell nn = lds_cell(s_q, own + RX), s = lds_cell(s_q, own - RX);
         pair_terms<1>(o, s, cv, t);
 #pragma unroll
-        for (int n = 0; n < 5; ++n) ay[n] = 0.0 + (two ? 1.0 : co0) * t[n];
+        for (int n = 0; n < 5; ++n) ay[n] = (two ? 1.0 : co0) * t[n];
         if (H == 2) {
           pair_terms<1>(nn, s, cv, t);
 #pragma unroll
@@ -543,7 +543,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
         const double ca = two16 && !rx ? 1.0 : co0;
         pair_terms_xy(rx, q, b, cv, t);
 #pragma unroll
-        for (int n = 0; n < 5; ++n) s_a[n][rslot] = 0.0 + ca * t[n];
+        for (int n = 0; n < 5; ++n) s_a[n][rslot] = ca * t[n];
       }
     }
     if (ring) {
@@ -608,7 +608,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
           f += s_e[n][pe];
           fy[n] = two ? fy[n] : f;
         }
-        if (n > 0) fy[n] += 0.5 * (s_e[NP + n - 1][pe - TX] + s_e[NP + n - 1][pe]);
+        if (n > 0) fy[n] = __builtin_fma(0.5, s_e[NP + n - 1][pe - TX] + s_e[NP + n - 1][pe], fy[n]);
       }
       if (tj > 0)
 #pragma unroll
@@ -623,7 +623,7 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
             g += s_e[n][E_HI + tid];
             f = two16 && isy ? f : g;
           }
-          if (n > 0) f += 0.5 * (s_e[NP + n - 1][elo] + s_e[NP + n - 1][E_HI + tid]);
+          if (n > 0) f = __builtin_fma(0.5, s_e[NP + n - 1][elo] + s_e[NP + n - 1][E_HI + tid], f);
           s_f[n][edst] = f;
         }
       }
