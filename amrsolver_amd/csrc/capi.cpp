@@ -2084,6 +2084,33 @@ int ensure_adjoint_level(amr_boxtab_s* bt, const amr_scheme_t& s) {
   return AMR_OK;
 }
 
+// Whether one marching kernel reverses a stage of this periodic level, and
+// its tiles: KEEP order 2/4, boxes that fill most lanes of 16x16 columns (the
+// passes gather a cell per lane of any box), and the plane count of least
+// estimated time.  A tile costs an iteration per plane plus two, 1.35 times as
+// long once CUs are shared.  Measured, 8 steps checkpointed every 3, tz 1, 2,
+// 4, 8 (passes): 24^3 976, 1076, 1342, 1896 us (1171); 96x48x40 1362, 1345,
+// 1489, 2063 (1845); 126x71x72 3768, 3401, 3304, 3288, tz 6 3084 (5728).
+bool march_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, const StageArgs& sa, FusedConfig* out) {
+  FusedConfig cfg{16, 16, 64};
+  if (!adj_march_supported(sch) || sa.box_dt || !fused_fits(bt, cfg)) return false;
+  const int64_t slots = 256 * adj_march_per_cu(sch);
+  double best = 0.0;
+  for (int tz : {64, 32, 16, 12, 8, 6, 4, 3, 2, 1}) {
+    cfg.tz = tz;
+    int64_t it = 0;
+    int mx = 0;
+    const int64_t n = tile_count(bt, cfg, &it, &mx);  // three iterations more than planes per tile
+    double t = mx - 1;
+    if (n > 256) t = 1.35 * std::max(t, n <= 4 * slots ? double((n + slots - 1) / slots) * t : double(it - n) / slots);
+    if (tz == 64 || t < best) {
+      best = t;
+      *out = cfg;
+    }
+  }
+  return true;
+}
+
 // Reverse of one stage: lam_sin (=|+=) stage terms of lam_out through the
 // RHS VJP at `sin` (ghost-filled); lam_s1 gets a lam_out (s1_mode 1: +=,
 // 2: =).  lam_sin and lam_s1 must not alias lam_out.
@@ -2091,13 +2118,20 @@ int adj_stage(amr_boxtab_s* bt, const amr_closures_t& cls, const amr_scheme_t& s
               DescSet* sin, DescSet* lam_out, const DescSet* lam_s1, const DescSet* lam_sin, bool acc,
               int s1_mode) {
   int rc;
-  if ((rc = ensure_unfused(bt, sch))) return rc;
-  if ((rc = ensure_adjoint(bt, sch))) return rc;
   const Closures c = make_closures(cls);
-  const FoldTasks& ft = bt->fold;
   const WrapArgs wa = wrap_args(bt, sin);
   // the domain-wide path needs lam_out as one periodic array as well
   const bool level = wa.on && wrap_ok(bt, lam_out);
+  if (FusedConfig cfg; level && march_path(bt, sch, sa, &cfg)) {
+    TileTable* tt;
+    if ((rc = get_tiles(bt, cfg, false, &tt))) return rc;
+    HIPCHK(launch_adj_march(sch, tt->d, tt->n, bt->bt.d_boxes, c, sa.sc, wa, sin->d, lam_out->d,
+                            lam_s1 ? lam_s1->d : nullptr, lam_sin->d, acc, lam_s1 ? s1_mode : 0, bt->ctx->stream));
+    return AMR_OK;
+  }
+  if ((rc = ensure_unfused(bt, sch))) return rc;
+  if ((rc = ensure_adjoint(bt, sch))) return rc;
+  const FoldTasks& ft = bt->fold;
   if (level && (rc = ensure_adjoint_level(bt, sch))) return rc;
   AdjWork aw = bt->aw;
   if (!level) aw.lq = aw.le = nullptr;

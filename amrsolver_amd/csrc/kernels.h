@@ -230,6 +230,7 @@ hipError_t launch_prims(const BoxTable& bt, const UnfusedWork& w, const Closures
 
 // Reverse mode of the KEEP + viscous RHS (adjoint.hip).  Workspace per box:
 // e = 16 comps on grow(bx,1) (viscous), g = NCONS comps on grow(bx,3).
+struct TileDev;
 struct AdjWork {
   Fab* e = nullptr;
   Fab* g = nullptr;
@@ -261,6 +262,14 @@ struct FoldTasks {
 hipError_t launch_adj_stage(const BoxTable& bt, const UnfusedWork& w, const AdjWork& aw, const Closures& c,
                             const amr_scheme_t& s, const StageArgs& sa, const WrapArgs& wa, const Fab* sin, const Fab* lam_out, const Fab* lam_s1, const Fab* lam_sin,
                             bool accumulate, int s1_mode, const FoldTasks& ft, hipStream_t st);
+// The same stage of a periodic level held as one array (wa.on, lam_out too) in
+// one kernel over tiles of 16x16 columns.
+bool adj_march_supported(const amr_scheme_t& s);
+int adj_march_per_cu(const amr_scheme_t& s);  // workgroups that a CU holds
+hipError_t launch_adj_march(const amr_scheme_t& s, const TileDev* tiles, int ntiles, const BoxDev* boxes,
+                            const Closures& c, const StageCoef& sc, const WrapArgs& wa, const Fab* sin,
+                            const Fab* lam_out, const Fab* lam_s1, const Fab* lam_sin, bool accumulate, int s1_mode,
+                            hipStream_t st);
 // Objective of the final state and its gradient lam (kind 0 kinetic energy,
 // kind 1 linear with weights); result[0] = J.
 hipError_t launch_objective(const BoxTable& bt, int kind, const Fab* st, const Fab* wts, const Fab* lam,
