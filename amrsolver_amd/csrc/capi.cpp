@@ -1164,14 +1164,15 @@ double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedC
 // self-loading form where there is one) unless they would be mostly idle,
 // with the plane count of least estimated time -- short tiles where a level
 // has too few columns to fill the chip (32x24x20 in 8 boxes: 8x8x64 took
-// 90 us a right-hand side, 16x16x4 takes 30).
+// 90 us a right-hand side, 16x16x4 takes 26, 16x16x1 14; order 6 on 40x47x33,
+// the CFL estimate included, 261, 70, 51).
 FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
   FusedConfig c{16, 16, 64};
   if (fused_self_supported(sch, 16, 16)) c.form = 1;
   if (!fused_fits(bt, c)) c = FusedConfig{8, 8, 64};
   double best = 0.0;
   FusedConfig out = c;
-  for (int tz : {64, 32, 16, 8, 4}) {
+  for (int tz : {64, 32, 16, 8, 4, 2, 1}) {
     c.tz = tz;
     const double t = tiling_time(bt, sch, c);
     if (tz == 64 || t < best) {

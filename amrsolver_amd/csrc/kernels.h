@@ -320,6 +320,7 @@ hipError_t launch_pack_valid(const BoxTable& bt, const Fab* src, int ncomp, cons
 // Reductions over valid cells.  `partial` holds at least reduce_partials()
 // doubles (x5 for totals); the result lands in result[0] (dt) or result[0..4].
 int reduce_blocks(const BoxTable& bt);
+constexpr int ESTDT_MAX_BLOCKS = 1024;  // partial minima of launch_estdt
 hipError_t launch_estdt(const BoxTable& bt, const Fab* st, const Closures& c, double* partial,
                         double* result, hipStream_t s);
 // per-box minimum of cns_estdt: result[b] for every box (estdt_box_blocks
