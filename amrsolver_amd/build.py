@@ -32,7 +32,7 @@ DEVICE = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-SOURCES = ["capi.cpp", "unfused.hip", "fused.hip", "fused_self.hip", "fill_reduce.hip", "adjoint.hip", "adjoint_march.hip", "dir_flux.hip", "tube_flux.hip", "regrid.hip",
+SOURCES = ["capi.cpp", "unfused.hip", "fused.hip", "fused_self.hip", "fused_keep6.hip", "fill_reduce.hip", "adjoint.hip", "adjoint_march.hip", "dir_flux.hip", "tube_flux.hip", "regrid.hip",
            "user_source.cpp"]
 
 

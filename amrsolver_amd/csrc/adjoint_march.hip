@@ -39,13 +39,6 @@ using namespace tile16;
 
 constexpr int OB = RB - NOUT;  // first thread of the halo cells that are not ring cells
 
-// Ends a section: nothing is scheduled across, and LDS values are read again
-// rather than held in registers (with them held the kernel spilled).
-__device__ __forceinline__ void section() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // The adjoint weights of the viscous cell fluxes (a, b, c: half the central
 // differences of the stage adjoint in x, y, z, components 1..4) turned into
 // the adjoints of the stresses.

@@ -655,8 +655,16 @@ bool launch_shape(const amr_scheme_t& s, const TileDev* tiles, int ntiles, const
                   hipStream_t st) {
   const bool v = s.rhs_visc != 0;
   if (s.order_keep == 6) {
-    if (v) launch_t<3, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-    else launch_t<3, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    if constexpr (TX == 16 && TY == 16) {
+      if (v) {
+        launch_fused_keep6(tiles, ntiles, boxes, c, co, sa, wa, cov, us, s1, sin, out, st);
+        return true;
+      }
+    } else if (v) {
+      launch_t<3, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+      return true;
+    }
+    launch_t<3, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   } else if (s.order_keep == 4) {
     if (v) launch_t<2, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
     else launch_t<2, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);

@@ -435,6 +435,10 @@ struct UncovSrc {
 constexpr int UNCOV_MAX_ZBLK = 32;
 bool fused_supported(const amr_scheme_t& s, int tx, int ty);
 // the self-loading form of the fused kernel (FusedConfig::form 1) applies
+// The viscous order 6 stage on tiles of 16x16 columns.
+hipError_t launch_fused_keep6(const TileDev* tiles, int ntiles, const BoxDev* boxes, const Closures& c,
+                              const double co[3], const StageArgs& sa, const WrapArgs& wa, const Cover& cov,
+                              const UncovSrc& us, const Fab* s1, const Fab* sin, const Fab* out, hipStream_t st);
 bool fused_self_supported(const amr_scheme_t& s, int tx, int ty);
 // bc 6 walls in y for the self-loading form: the domain's y bounds and which
 // of them are walls (tiles per box; box boundaries decide which tiles touch).

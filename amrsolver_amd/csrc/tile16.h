@@ -63,5 +63,12 @@ __device__ __forceinline__ double uniform(double v) {
                           __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
+// Ends a section: nothing is scheduled across, and LDS values are read again
+// rather than held in registers (with them held the kernel spilled).
+__device__ __forceinline__ void section() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace tile16
 }  // namespace amr
