@@ -224,6 +224,7 @@ __device__ __forceinline__ void pencil_cell(const WenoBrick& W, const BoxDev& bx
 // Fv(right)) per component (CNS_hydro_K.h:254-261, the reference's operand
 // order).  Cells beyond the box (faces of overhanging lanes, whose fluxes
 // are never used) are clamped into the viscous fluxes' grown-by-one extent.
+// There is no mass component.
 template <int D, int FX>
 __device__ __forceinline__ void add_visc_face(const WenoBrick& W, const BoxDev& bx, const Fab& P, int f,
                                               double F[5]) {
@@ -235,7 +236,7 @@ __device__ __forceinline__ void add_visc_face(const WenoBrick& W, const BoxDev& 
   brick_ijk<D>(xl, bl, W.c, il, jl, kl);
   brick_ijk<D>(xr, br, W.c, ir, jr, kr);
 #pragma unroll
-  for (int n = 0; n < 5; ++n) F[n] += 0.5 * (P(il, jl, kl, n) + P(ir, jr, kr, n));
+  for (int n = 1; n < 5; ++n) F[n] += 0.5 * (P(il, jl, kl, n) + P(ir, jr, kr, n));
 }
 
 template <int D, int LAST>
