@@ -156,13 +156,10 @@ k_fused_self(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const int cell = load_cell(s);
-    int x = T.i0 - HX + cell % RX, y = T.j0 - HX + cell / RX;
+    int x = min(T.i0 - HX + cell % RX, xcap), y = min(T.j0 - HX + cell / RX, ycap);
     if (wa.on) {
       x = x < wa.lo[0] ? x + wa.len[0] : (x >= wa.lo[0] + wa.len[0] ? x - wa.len[0] : x);
       y = y < wa.lo[1] ? y + wa.len[1] : (y >= wa.lo[1] + wa.len[1] ? y - wa.len[1] : y);
-    } else {
-      x = min(x, xcap);
-      y = min(y, ycap);
     }
     loff[s] = x + y * int(S.js);
   }
@@ -626,7 +623,7 @@ hipError_t launch_fused_self(const amr_scheme_t& s, const FusedConfig& cfg, cons
                              const Closures& c, const StageArgs& sa, const Fab* s1, const Fab* sin, const Fab* out,
                              hipStream_t st, const NbMap& nbm, const WallRows& wr) {
   if (!fused_self_supported(s, cfg.tx, cfg.ty) || (nbm.on && us.on) ||
-      (wr.on && (nbm.on || us.on || wa.on || cov.on)))
+      (wr.on && (nbm.on || us.on || cov.on)))
     return hipErrorInvalidValue;
   double co[3];
   keep_coefficients(s.order_keep, co);
