@@ -3468,7 +3468,7 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
         // short tiles only where longer ones leave the chip idle
         if (tz < 16 && tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz}) >= 1024) continue;
         if (!(fused_supported(*sch, c.tx, c.ty) && fused_fits(bt, c, !box_tiles))) continue;
-        // the self-loading form where there is one (TGV 256^3, KEEP4: 0.68
+        // the self-loading form where there is one (TGV 256^3, KEEP4: 0.67
         // ms a stage against 0.77; KEEP2 0.59 against 0.64), which also
         // leaves 32x8 columns behind (1.2 ms); next to walls only that form
         if (self16) {

@@ -562,9 +562,9 @@ hipError_t launch_unfused_stage(const BoxTable& bt, const UnfusedWork& w, const 
   const Region g3 = grown(NGHOST), nod = nodal(), g1 = grown(1), g0 = grown(0);
   // WENO or MUSCL: directional passes from the conserved state, each
   // forming what it needs of its pencil in LDS; with viscous terms the
-  // cell-centred viscous fluxes are computed first (primitives on grow(bx,3),
-  // ViscousFluxes on grow(bx,1), the wall rows' own fluxes next to bc 6
-  // walls) and each pass adds their face averages
+  // cell-centred viscous fluxes are computed first (ViscousFluxes on
+  // grow(bx,1); next to bc 6 walls from primitives on grow(bx,3), with the
+  // wall rows' own fluxes) and each pass adds their face averages
   if (!faces && !sa.rhs_only && s.rhs_euler && (s.flux_euler == 2 || s.flux_euler == 0) && !s.art_diss &&
       w.weno.d[0] != nullptr) {
     if (!s.rhs_visc && w.tube.d)
