@@ -210,14 +210,38 @@ __device__ __forceinline__ double cell_estdt(const Fab& u, int i, int j, int k, 
   return dmin(dtx, dmin(dty, dtz));
 }
 
+// Minimum over the workgroup, in every thread: within a wave by lane
+// exchanges, then over the waves (one barrier instead of nine).
 __device__ __forceinline__ double block_min(double v, double* sm) {
-  sm[threadIdx.x] = v;
+  for (int d = 32; d > 0; d >>= 1) v = dmin(v, __shfl_xor(v, d));
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int s = RBLK / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] = dmin(sm[threadIdx.x], sm[threadIdx.x + s]);
-    __syncthreads();
+  v = sm[0];
+#pragma unroll
+  for (int w = 1; w < RBLK / 64; ++w) v = dmin(v, sm[w]);
+  return v;
+}
+
+// Smallest time step of the cells first, first + stride, ... of a box.  Cell
+// numbers fit 32 bits (a 64-bit division is some 100 instructions, and a
+// small box's estimate is one cell's latency) except in boxes of 2^31 cells.
+template <class Int>
+__device__ __forceinline__ double strided_estdt(const BoxDev& bx, const Fab& u, const Closures& c, Int first,
+                                                Int stride, Int nx, Int ny, Int n, double dt) {
+  for (Int t = first; t < n; t += stride) {
+    const Int r = t / nx, k = r / ny;
+    dt = dmin(dt, cell_estdt(u, bx.lo[0] + int(t - r * nx), bx.lo[1] + int(r - k * ny), bx.lo[2] + int(k), c, bx.dx[0],
+                             bx.dx[1], bx.dx[2]));
   }
-  return sm[0];
+  return dt;
+}
+__device__ __forceinline__ double box_estdt(const BoxDev& bx, const Fab& u, const Closures& c, double dt) {
+  const int nx = bx.hi[0] - bx.lo[0] + 1, ny = bx.hi[1] - bx.lo[1] + 1, nz = bx.hi[2] - bx.lo[2] + 1;
+  const int64_t n = int64_t(nx) * ny * nz, first = int64_t(blockIdx.x) * RBLK + threadIdx.x;
+  const int64_t stride = int64_t(gridDim.x) * RBLK;
+  if (n + stride < (int64_t(1) << 32))
+    return strided_estdt<unsigned>(bx, u, c, unsigned(first), unsigned(stride), nx, ny, unsigned(n), dt);
+  return strided_estdt<int64_t>(bx, u, c, first, stride, nx, ny, n, dt);
 }
 
 // per-box minimum: blockIdx.y = box, partial[box * gridDim.x + blockIdx.x]
@@ -233,17 +257,7 @@ __global__ void __launch_bounds__(RBLK) k_estdt_boxes(const BoxDev* boxes, const
   }
   const BoxDev bx = boxes[b];
   const Fab u = st[b];
-  double dt = 1.79769313486231570815e+308;
-  int nx = bx.hi[0] - bx.lo[0] + 1, ny = bx.hi[1] - bx.lo[1] + 1, nz = bx.hi[2] - bx.lo[2] + 1;
-  int64_t n = int64_t(nx) * ny * nz;
-  for (int64_t t = int64_t(blockIdx.x) * RBLK + threadIdx.x; t < n; t += int64_t(gridDim.x) * RBLK) {
-    int i = bx.lo[0] + int(t % nx);
-    int64_t r = t / nx;
-    int j = bx.lo[1] + int(r % ny);
-    int k = bx.lo[2] + int(r / ny);
-    dt = dmin(dt, cell_estdt(u, i, j, k, c, bx.dx[0], bx.dx[1], bx.dx[2]));
-  }
-  double m = block_min(dt, sm);
+  const double m = block_min(box_estdt(bx, u, c, 1.79769313486231570815e+308), sm);
   if (threadIdx.x == 0) partial[size_t(b) * gridDim.x + blockIdx.x] = m;
 }
 
@@ -257,25 +271,12 @@ __global__ void __launch_bounds__(RBLK) k_min_boxes(const double* partial, int n
 
 // Minimum over all boxes: workgroup (x, y) takes chunk x of boxes y, y +
 // gridDim.y, ...  With every workgroup walking every box the descriptor loads
-// of the boxes stood in a row: 12.4 us for 8 boxes of 16x12x10, now 4.6.
+// of the boxes stood in a row: 12.4 us for 8 boxes of 16x12x10, now 4.3.
 __global__ void __launch_bounds__(RBLK) k_estdt(const BoxDev* boxes, int nbox, const Fab* st,
                                                 Closures c, double* partial) {
   __shared__ double sm[RBLK];
   double dt = 1.79769313486231570815e+308;
-  for (int b = blockIdx.y; b < nbox; b += gridDim.y) {
-    const BoxDev bx = boxes[b];
-    const double dx0 = bx.dx[0], dx1 = bx.dx[1], dx2 = bx.dx[2];
-    const Fab u = st[b];
-    int nx = bx.hi[0] - bx.lo[0] + 1, ny = bx.hi[1] - bx.lo[1] + 1, nz = bx.hi[2] - bx.lo[2] + 1;
-    int64_t n = int64_t(nx) * ny * nz;
-    for (int64_t t = int64_t(blockIdx.x) * RBLK + threadIdx.x; t < n; t += int64_t(gridDim.x) * RBLK) {
-      int i = bx.lo[0] + int(t % nx);
-      int64_t r = t / nx;
-      int j = bx.lo[1] + int(r % ny);
-      int k = bx.lo[2] + int(r / ny);
-      dt = dmin(dt, cell_estdt(u, i, j, k, c, dx0, dx1, dx2));
-    }
-  }
+  for (int b = blockIdx.y; b < nbox; b += gridDim.y) dt = box_estdt(boxes[b], st[b], c, dt);
   const double m = block_min(dt, sm);
   if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = m;
 }
@@ -284,13 +285,8 @@ __global__ void __launch_bounds__(RBLK) k_min_final(const double* partial, int n
   __shared__ double sm[RBLK];
   double v = 1.79769313486231570815e+308;
   for (int t = threadIdx.x; t < n; t += RBLK) v = dmin(v, partial[t]);
-  sm[threadIdx.x] = v;
-  __syncthreads();
-  for (int s = RBLK / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] = dmin(sm[threadIdx.x], sm[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) result[0] = sm[0];
+  v = block_min(v, sm);
+  if (threadIdx.x == 0) result[0] = v;
 }
 
 // Conserved totals: per-block sums of the five components (fixed reduction
@@ -623,7 +619,9 @@ int estdt_box_blocks(const BoxTable& bt) {
   int64_t mx = 1;
   for (auto& b : bt.h_boxes)
     mx = std::max<int64_t>(mx, int64_t(b.hi[0] - b.lo[0] + 1) * (b.hi[1] - b.lo[1] + 1) * (b.hi[2] - b.lo[2] + 1));
-  int64_t nb = (mx + RBLK * 8 - 1) / (RBLK * 8);
+  // eight cells a lane, but up to eight workgroups a box before a lane takes a
+  // second cell: a Sod step's estimate is one cell's latency (5.9 us, now 3.6)
+  const int64_t nb = std::max<int64_t>((mx + RBLK * 8 - 1) / (RBLK * 8), std::min<int64_t>((mx + RBLK - 1) / RBLK, 8));
   return int(std::max<int64_t>(1, std::min<int64_t>(nb, 64)));
 }
 
