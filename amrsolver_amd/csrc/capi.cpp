@@ -273,6 +273,8 @@ struct amr_boxtab_s {
   int uw_kinds = 0;  // bitmask of allocated kinds
   UnfusedWork uw;
   std::vector<void*> uw_tables;
+  TubeWork tube;  // brick table of the tube stages (d null: not such a table, or not built yet)
+  bool tube_built = false;
   // advance workspace (two ghosted state copies mirroring the caller layout)
   double* ws_mem[2] = {nullptr, nullptr};
   std::vector<amr_fab_t> ws_fabs[2];
@@ -853,13 +855,18 @@ enum { UW_PRIMS = 1, UW_VISC = 2, UW_WENO = 4, UW_SLOPE = 8, UW_JST = 16 };
 // they fill less than a few rounds of the chip (one workgroup a CU): above
 // that the long bricks' throughput wins.
 int build_tube(amr_boxtab_s* bt) {
-  if (!bt->d_xside) return AMR_OK;
+  if (bt->tube_built) return AMR_OK;
+  bool is = bt->d_xside != nullptr;
   int64_t short_bricks = 0;
   for (auto& B : bt->bt.h_boxes) {
-    if (B.hi[1] - B.lo[1] != 3 || B.hi[2] - B.lo[2] != 3) return AMR_OK;
+    is = is && B.hi[1] - B.lo[1] == 3 && B.hi[2] - B.lo[2] == 3;
     short_bricks += (B.hi[0] - B.lo[0] + TUBE_SPLIT_NX) / TUBE_SPLIT_NX;
   }
-  TubeWork& w = bt->uw.tube;
+  if (!is) {
+    bt->tube_built = true;
+    return AMR_OK;
+  }
+  TubeWork& w = bt->tube;
   w.split = short_bricks <= TUBE_SPLIT_MAX;
   const int most = w.split ? TUBE_SPLIT_NX : TUBE_NX;
   std::vector<TubeBrick> h;
@@ -877,8 +884,8 @@ int build_tube(amr_boxtab_s* bt) {
   }
   HIPCHK(hipMalloc(&w.d, sizeof(TubeBrick) * h.size()));
   HIPCHK(hipMemcpy(w.d, h.data(), sizeof(TubeBrick) * h.size(), hipMemcpyHostToDevice));
-  bt->uw_tables.push_back(w.d);
   w.n = int(h.size());
+  bt->tube_built = true;
   return AMR_OK;
 }
 
@@ -971,7 +978,6 @@ int ensure_unfused(amr_boxtab_s* bt, const amr_scheme_t& s) {
       bt->uw.weno.n[d] = n;
     }
     bt->uw.weno.xside = bt->d_xside;
-    if (int rc = build_tube(bt)) return rc;
   }
   bt->uw_kinds = need;
   return AMR_OK;
@@ -980,6 +986,17 @@ int ensure_unfused(amr_boxtab_s* bt, const amr_scheme_t& s) {
 // Schemes the directional flux passes run (unfused.hip).
 bool dir_flux_scheme(const amr_scheme_t& s) {
   return s.rhs_euler && (s.flux_euler == 2 || s.flux_euler == 0) && !s.rhs_visc && !s.art_diss;
+}
+
+// Whether a stage of the table is one tube kernel, which needs no workspace
+// (512 1D problems of 8.65M cells: 12 GB of primitives, fluxes and splits,
+// whose clearing took 2.6 ms of a new batch's first call).
+int tube_path(amr_boxtab_s* bt, const amr_scheme_t& s, bool* yes) {
+  *yes = false;
+  if (!dir_flux_scheme(s) || (s.rhs_source && bt->usrc_fn)) return AMR_OK;
+  if (int rc = build_tube(bt)) return rc;
+  *yes = bt->tube.d != nullptr;
+  return AMR_OK;
 }
 
 std::string scheme_key(const amr_scheme_t& s) {
@@ -1715,8 +1732,14 @@ int do_stage(amr_boxtab_s* bt, const amr_closures_t& cls, const amr_scheme_t& sc
     return AMR_OK;
   }
   if (uncov_u0) return fail(AMR_ERR_ARG, "internal: uncovered ghost cells from U^n requested off the fused path");
-  int rc = ensure_unfused(bt, sch);
+  bool tube = false;
+  int rc = tube_path(bt, sch, &tube);
   if (rc) return rc;
+  if (tube) {
+    HIPCHK(launch_tube(sch.flux_euler, bt->tube, bt->bt.d_boxes, c, sa, dsin->d, s1, dout->d, bt->d_xside, st));
+    return AMR_OK;
+  }
+  if ((rc = ensure_unfused(bt, sch))) return rc;
   HIPCHK(launch_unfused_stage(bt->bt, bt->uw, c, sch, sa, bt->wall_args, s1, dsin->d, dout->d, st));
   return AMR_OK;
 }
@@ -1918,7 +1941,9 @@ int prepare_step_tables(amr_boxtab_s* bt, const amr_scheme_t& sch, const amr_fab
   TileTable* tt = nullptr;
   if (fused && fused_fits(bt, cfg) && (rc = get_tiles(bt, cfg, false, &tt))) return rc;
   if (fused && bt->cover.on && (rc = get_tiles(bt, cfg, true, &tt))) return rc;
-  if (!(fused && fused_fits(bt, cfg)) && (rc = ensure_unfused(bt, sch))) return rc;
+  bool tube = false;
+  if (!(fused && fused_fits(bt, cfg)) && ((rc = tube_path(bt, sch, &tube)) || (!tube && (rc = ensure_unfused(bt, sch)))))
+    return rc;
   return AMR_OK;
 }
 
@@ -2638,6 +2663,7 @@ int amr_boxtab_destroy(amr_boxtab_t bt) {
   bt->descs.clear();
   if (bt->uw_mem) (void)hipFree(bt->uw_mem);
   for (void* p : bt->uw_tables) (void)hipFree(p);
+  if (bt->tube.d) (void)hipFree(bt->tube.d);
   for (int w = 0; w < 2; ++w)
     if (bt->ws_mem[w]) (void)hipFree(bt->ws_mem[w]);
   if (bt->d_uncov) (void)hipFree(bt->d_uncov);

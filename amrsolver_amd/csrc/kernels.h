@@ -81,7 +81,6 @@ void weno_bricks(const BoxTable& bt, int d, const int* wrap, WenoBrick* out);
 // nbox Fab each).
 struct UnfusedWork {
   WenoWork weno;            // brick tables of the directional flux passes
-  TubeWork tube;            // brick table of the tube stages (d null: not such a table)
   Fab* prims = nullptr;     // NPRIM comps on grow(bx,3)
   Fab* nf[3] = {};          // NCONS comps on [lo, hi+1]^3
   Fab* pv[3] = {};          // NCONS comps on grow(bx,1)   (viscous)

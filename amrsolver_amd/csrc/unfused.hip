@@ -567,8 +567,6 @@ hipError_t launch_unfused_stage(const BoxTable& bt, const UnfusedWork& w, const 
   // wall rows' own fluxes) and each pass adds their face averages
   if (!faces && !sa.rhs_only && s.rhs_euler && (s.flux_euler == 2 || s.flux_euler == 0) && !s.art_diss &&
       w.weno.d[0] != nullptr) {
-    if (!s.rhs_visc && w.tube.d)
-      return launch_tube(s.flux_euler, w.tube, B, c, sa, sin, s1, out, w.weno.xside, st);
     if (!s.rhs_visc) return launch_dir_flux(s.flux_euler, w.weno, B, c, sa, sin, w.nf[0], s1, out, st);
     if (w.pv[0] != nullptr) {
       if (wa.nvisc_blk == 0) {
