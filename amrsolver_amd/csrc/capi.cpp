@@ -318,6 +318,9 @@ struct amr_boxtab_s {
   hipStream_t aux = nullptr;  // second stream (adjoint runs: recompute beside the reverse sweep)
   // autotuned tiling per scheme key for this box table
   std::map<std::string, FusedConfig> tuned;
+  // estimated tilings of this table per scheme, forward and reverse (they
+  // depend on the boxes, which do not change, and the scheme alone)
+  mutable std::map<std::array<int, 6>, FusedConfig> estimated;
   // source added to dSdt for schemes with rhs_source = 1 (amr_set_source)
   std::unique_ptr<DescSet> src;
   // ghost cells of each box covered by no box of the level (coarse-fine
@@ -1179,6 +1182,16 @@ double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedC
   return 1.35 * std::max(rounds, double(mx));
 }
 
+// Plane counts of tiles that the estimates choose from: dense where tiles are
+// short, since one plane fewer is then a tenth of the time (the channel
+// 96x128x64 has 48 columns a piece: 8 planes a tile leave a quarter of the
+// slots empty, 7 fill them).
+constexpr int TILE_PLANES[] = {64, 48, 32, 24, 20, 16, 14, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2, 1};
+
+std::array<int, 6> estimate_key(const amr_scheme_t& s, int reverse) {
+  return {s.rhs_euler, s.rhs_visc, s.flux_euler, s.order_keep, s.art_diss, reverse};
+}
+
 // The tiling of a table that has not been autotuned: 16x16 columns (in the
 // self-loading form where there is one) unless they would be mostly idle,
 // with the plane count of least estimated time -- short tiles where a level
@@ -1186,12 +1199,14 @@ double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedC
 // 90 us a right-hand side, 16x16x4 takes 26, 16x16x1 14; order 6 on 40x47x33,
 // the CFL estimate included, 261, 70, 51).
 FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
+  const auto known = bt->estimated.find(estimate_key(sch, 0));
+  if (known != bt->estimated.end()) return known->second;
   FusedConfig c{16, 16, 64};
   if (fused_self_supported(sch, 16, 16)) c.form = 1;
   if (!fused_fits(bt, c)) c = FusedConfig{8, 8, 64};
   double best = 0.0;
   FusedConfig out = c;
-  for (int tz : {64, 32, 16, 8, 4, 2, 1}) {
+  for (int tz : TILE_PLANES) {
     c.tz = tz;
     const double t = tiling_time(bt, sch, c);
     if (tz == 64 || t < best) {
@@ -1199,6 +1214,7 @@ FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
       out = c;
     }
   }
+  bt->estimated[estimate_key(sch, 0)] = out;
   return out;
 }
 
@@ -2166,9 +2182,14 @@ int ensure_adjoint_level(amr_boxtab_s* bt, const amr_scheme_t& s) {
 bool march_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, const StageArgs& sa, FusedConfig* out) {
   FusedConfig cfg{16, 16, 64};
   if (!adj_march_supported(sch) || sa.box_dt || !fused_fits(bt, cfg)) return false;
+  const auto known = bt->estimated.find(estimate_key(sch, 1));
+  if (known != bt->estimated.end()) {
+    *out = known->second;
+    return true;
+  }
   const int64_t slots = 256 * adj_march_per_cu(sch);
   double best = 0.0;
-  for (int tz : {64, 32, 16, 12, 8, 6, 4, 3, 2, 1}) {
+  for (int tz : TILE_PLANES) {
     cfg.tz = tz;
     int64_t it = 0;
     int mx = 0;
@@ -2180,6 +2201,7 @@ bool march_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, const StageArgs
       *out = cfg;
     }
   }
+  bt->estimated[estimate_key(sch, 1)] = *out;
   return true;
 }
 
@@ -3487,14 +3509,17 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
   std::vector<FusedConfig> cand;
   const bool self16 = fused_self_supported(*sch, 16, 16) && fused_fits(bt, FusedConfig{16, 16, 16});
   const int shapes[3][2] = {{16, 16}, {32, 8}, {8, 8}};
-  const int tzs[8] = {4, 8, 16, 24, 32, 48, 64, 128};
+  // the usual plane counts and the one of least estimated time
+  std::vector<int> tzs = {4, 8, 16, 24, 32, 48, 64, 128};
+  const int est = default_config(bt, *sch).tz;
+  if (std::find(tzs.begin(), tzs.end(), est) == tzs.end()) tzs.push_back(est);
   for (int box_tiles = level ? 0 : 1; box_tiles <= 1; ++box_tiles)
     for (auto& sh : shapes)
       for (int tz : tzs) {
         FusedConfig c{sh[0], sh[1], tz, box_tiles};
         if (tz > 2 * (box_tiles ? maxz : maxz_level) && tz != 16) continue;
         // short tiles only where longer ones leave the chip idle
-        if (tz < 16 && tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz}) >= 1024) continue;
+        if (tz < 16 && tz != est && tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz}) >= 1024) continue;
         if (!(fused_supported(*sch, c.tx, c.ty) && fused_fits(bt, c, !box_tiles))) continue;
         // the self-loading form where there is one (TGV 256^3, KEEP4: 0.67
         // ms a stage against 0.77; KEEP2 0.59 against 0.64), which also
