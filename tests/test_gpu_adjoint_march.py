@@ -56,3 +56,29 @@ def test_march_matches_passes(ctx, n, mg, visc, order):
                 for a, b in zip(got["level"], got["boxes"]):
                     for k in range(5):
                         assert np.max(np.abs(a[k] - b[k])) <= 1e-12 * np.max(np.abs(b[k])), f"component {k}"
+
+
+def test_march_with_outputs_per_box(ctx):
+    """State and stage adjoint in one array, the arrays that receive the result
+    one per box: the same bits as with all in one array."""
+    from amrsolver_amd import level as L
+    n, mg = (48, 32, 20), (32, 16, 12)
+    cls = P.closures_scaled_sutherland(0.02, T0=300.0)
+    g = P.geom(n, (0.0, 0.0, 0.0), (1.0, 0.8, 0.7), (1, 1, 1))
+    lev = L.Level(g, P.decompose(n, mg), cls, P.scheme(flux_euler=1, order_keep=4, visc=True), ctx=ctx)
+    u = P.smooth_random_state(cls, n, 5)
+    rng = np.random.default_rng(18)
+    lam, s0, s1 = (rng.standard_normal(u.shape) for _ in range(3))
+    S, Lo = lev.new_state(), lev.new_state(ng=0)
+    S.upload(u)
+    lev.fill_patch(S)
+    Lo.upload(lam)
+    got = []
+    for layout in ("level", "boxes"):
+        print(f"case march outputs {layout}", flush=True)
+        Li, L1 = (lev.new_state(layout=layout, ng=0) for _ in range(2))
+        Li.upload(s0)
+        L1.upload(s1)
+        lev.vjp_stage(0, 0.75, 0.25, 1.0, 2e-2, S, Lo, L1, Li, accumulate=True)
+        got.append((Li.download(), L1.download()))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
