@@ -233,6 +233,7 @@ struct CfTable {
   InterpTask* d_interp = nullptr;
   TaskBlock* d_interp_blk = nullptr;
   int ninterp_blk = 0;
+  int ninterp = 0;            // interpolation tasks
   int64_t ninterp_cells = 0;  // coarse cells (lanes) of the interpolation tasks
   CopyTask* d_avg = nullptr;
   TaskBlock* d_avg_blk = nullptr;
@@ -2908,7 +2909,8 @@ int build_cf_interp(amr_boxtab_s* F, amr_boxtab_s* C, int r, CfTable* t) {
     HIPCHK(hipMemcpy(t->d_interp, tasks.data(), sizeof(InterpTask) * tasks.size(), hipMemcpyHostToDevice));
   }
   t->ninterp_cells = ncell;
-  rc = upload_blocks(tasks, &t->d_interp_blk, &t->ninterp_blk);
+  t->ninterp = int(tasks.size());
+  rc = upload_packed_blocks(tasks, ncell, &t->d_interp_blk, &t->ninterp_blk);
   if (rc) return rc;
   t->interp_built = true;
   return AMR_OK;
@@ -2983,7 +2985,7 @@ int fill_two_levels(amr_boxtab_t fine, amr_boxtab_t crse, int ratio, double a_ol
   if (same_level) HIPCHK(launch_fill_copy(tk->d_copy, tk->ncopy, tk->d_copy_blk, tk->ncopy_blk, dsf->d, st));
   const bool blend = use_old && use_new;
   const Fab* c0 = use_old ? d0->d : d1->d;
-  HIPCHK(launch_interp_cf(t->d_interp, t->d_interp_blk, t->ninterp_blk, c0, blend ? d1->d : c0, blend, a_old,
+  HIPCHK(launch_interp_cf(t->d_interp, t->ninterp, t->d_interp_blk, t->ninterp_blk, c0, blend ? d1->d : c0, blend, a_old,
                           b_new, ratio, dsf->d, st));
   return enqueue_fill(fine, dsf, true, nullptr, width);
 }
@@ -3121,14 +3123,14 @@ int amr_regrid_fill(amr_boxtab_t fine_new, amr_boxtab_t fine_old, const amr_fab_
     HIPCHK(hipMalloc(&dint.p, sizeof(InterpTask) * itasks.size()));
     HIPCHK(hipMemcpy(dint.p, itasks.data(), sizeof(InterpTask) * itasks.size(), hipMemcpyHostToDevice));
   }
-  if ((rc = upload_blocks(itasks, &dint_blk.p, &nint_blk))) return rc;
+  if ((rc = upload_packed_blocks(itasks, ninterp, &dint_blk.p, &nint_blk))) return rc;
   hipStream_t st = fine_new->ctx->stream;
   if (ncopy_blk) HIPCHK(launch_copy_regions(dcopy.p, dcopy_blk.p, ncopy_blk, dold->d, dn->d, nullptr, st));
   if (nint_blk) {
     const bool blend = use_old && use_new;
     const Fab* c0 = use_old ? d0->d : d1->d;
-    HIPCHK(launch_interp_cf(dint.p, dint_blk.p, nint_blk, c0, blend ? d1->d : c0, blend, a_old, b_new, ratio, dn->d,
-                            st));
+    HIPCHK(launch_interp_cf(dint.p, int(itasks.size()), dint_blk.p, nint_blk, c0, blend ? d1->d : c0, blend, a_old,
+                            b_new, ratio, dn->d, st));
   }
   // the task lists are freed on return
   HIPCHK(hipStreamSynchronize(st));

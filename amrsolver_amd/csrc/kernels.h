@@ -298,8 +298,8 @@ struct InterpTask {
   int sh[3];
   int64_t start;
 };
-hipError_t launch_interp_cf(const InterpTask* tasks, const TaskBlock* blocks, int nblk, const Fab* c0, const Fab* c1,
-                            bool blend, double a, double b, int r, const Fab* fine, hipStream_t st);
+hipError_t launch_interp_cf(const InterpTask* tasks, int ntask, const TaskBlock* blocks, int nblk, const Fab* c0,
+                            const Fab* c1, bool blend, double a, double b, int r, const Fab* fine, hipStream_t st);
 // Coarse cells under fine boxes := mean of their r^3 children: per task,
 // dst = coarse box, src = fine box, lo/hi = coarse cells.
 hipError_t launch_avg_down(const CopyTask* tasks, const TaskBlock* blocks, int nblk, const Fab* fine,
