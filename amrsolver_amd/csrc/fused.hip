@@ -71,9 +71,12 @@ struct Cfg {
 // otherwise take registers past 256 (into AGPRs) rather than reuse them,
 // halving the occupancy.  Order 6 holds more (six pairs per x/y face, two
 // more z carries): one wave per SIMD with up to 512 registers rather than
-// spills to scratch memory.
+// spills to scratch memory.  Three waves for inviscid order 2 with neighbour
+// reads of equal strides, which fits 168 registers without a spill only when
+// asked to (left at two it took 174: 128x100x100 in boxes of 64x20x10 224 us
+// a step, at three 210; with a source it spills at three).
 template <int H, bool VISC, int TX, int TY, bool UCS, bool SRC, int NB>
-__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H == 3 ? 1 : 2))) k_fused(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes,
+__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H == 3 ? 1 : (H == 1 && !VISC && TX == 16 && !SRC && NB == 2 ? 3 : 2)))) k_fused(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes,
                                                      Closures c, double co0, double co1, double co2, StageArgs sa,
                                                      WrapArgs wa, Cover cov, UncovSrc us, NbMap nbm,
                                                      const Fab* __restrict__ s1f, const Fab* __restrict__ sinf,
