@@ -70,3 +70,8 @@ def test_inviscid_order_2_with_neighbour_reads_keeps_three_waves(kernels):
     224 us a step, at three 209."""
     k = kernels["k_fused<1, false, 16, 16, false, false, 2>"]
     assert _waves(k) >= 3 and k[".vgpr_spill_count"] == 0
+
+
+def test_pass_structured_order_4_keeps_to_four_waves(kernels):
+    """Five waves (96 registers or fewer) take 60 us on 96^3, four 57."""
+    assert _waves(kernels["k_keep<2>"]) == 4
