@@ -658,16 +658,10 @@ bool launch_shape(const amr_scheme_t& s, const TileDev* tiles, int ntiles, const
                   hipStream_t st) {
   const bool v = s.rhs_visc != 0;
   if (s.order_keep == 6) {
-    if constexpr (TX == 16 && TY == 16) {
-      if (v) {
-        launch_fused_keep6(tiles, ntiles, boxes, c, co, sa, wa, cov, us, s1, sin, out, st);
-        return true;
-      }
-    } else if (v) {
-      launch_t<3, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
-      return true;
-    }
-    launch_t<3, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    // viscous order 6 on 16x16 columns is launch_fused_keep6's
+    if (!v) launch_t<3, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
+    else if constexpr (TX == 16) return false;
+    else launch_t<3, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
   } else if (s.order_keep == 4) {
     if (v) launch_t<2, true, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
     else launch_t<2, false, TX, TY>(tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
@@ -698,6 +692,8 @@ hipError_t launch_fused_stage(const amr_scheme_t& s, const FusedConfig& cfg, con
   if ((nbm.on && (us.on || s.order_keep > 4)) || wr.on) return hipErrorInvalidValue;
   double co[3];
   keep_coefficients(s.order_keep, co);
+  if (s.order_keep == 6 && s.rhs_visc && cfg.tx == 16 && cfg.ty == 16)
+    return launch_fused_keep6(tiles, ntiles, boxes, c, co, sa, wa, cov, us, s1, sin, out, st);
   bool ok = false;
   if (cfg.tx == 16 && cfg.ty == 16)
     ok = launch_shape<16, 16>(s, tiles, ntiles, boxes, c, co, sa, wa, cov, us, nbm, s1, sin, out, st);
