@@ -194,10 +194,10 @@ struct Hierarchy {
       check(amr_fill_boundary(lev[0].bt, S.fabs.data()), "amr_fill_boundary");
       return;
     }
-    if (ngrow[l] == 0) {  // the fused stage kernel reads two ghost layers, the others three
+    if (ngrow[l] == 0) {  // the fused stage kernel of order 2 or 4 reads two ghost layers, the others three
       int32_t info[6];
       check(amr_step_plan(lev[l].bt, &sch, S.fabs.data(), info), "amr_step_plan");
-      ngrow[l] = info[3] != 0 ? 2 : 3;
+      ngrow[l] = info[3] != 0 && sch.order_keep <= 4 ? 2 : 3;
     }
     double a, b;
     cf_weights(t0[l - 1], t1[l - 1], t, &a, &b);

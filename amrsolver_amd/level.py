@@ -626,11 +626,11 @@ class Hierarchy:
         L = self.levels[lev]
         key = (lev, id(S))
         if key not in self.direct:
-            # the fused stage kernel reads two ghost layers, the others three;
-            # tiles per box may read the other boxes' cells themselves (decided
-            # per stage input)
+            # the fused stage kernel reads two ghost layers (three at order 6),
+            # the others three; tiles per box may read the other boxes' cells
+            # themselves (decided per stage input)
             plan = L.step_plan(S)
-            self.ngrow[lev] = 2 if plan["tiles"] != "passes" else 3
+            self.ngrow[lev] = 2 if plan["tiles"] != "passes" and L.scheme.order_keep <= 4 else 3
             self.direct[key] = plan["direct_neighbours"]
         direct = stage and self.direct[key]
         if lev == 0:

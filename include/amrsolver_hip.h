@@ -129,7 +129,8 @@ int amr_fill_boundary(amr_boxtab_t bt, const amr_fab_t* fabs);
  * alone within 1e-3 (t1 - t0) of its time), by conservative linear
  * interpolation; physical BCs.  Only the `ngrow` (1..3) ghost layers next to
  * each box are filled, as FillPatch's nghost argument does (the fused stage
- * kernel of amr_rk_stage reads 2; the other schemes need 3).  `crse` is the
+ * kernel of amr_rk_stage reads 2 at KEEP order 2 and 4; order 6 and the other
+ * schemes need 3).  `crse` is the
  * coarse level's box table,
  * `fine` this level's; fine_state needs ng >= 3, the coarse states ng >= 1
  * with their ghost cells filled (amr_fill_boundary or amr_fill_two_levels of
