@@ -620,9 +620,11 @@ class Hierarchy:
         return self.cur[lev].download()
 
     def _fill(self, lev, S, t, stage=False):
-        """Ghost cells of level lev's state S at time t; a stage input of a
-        level whose fused stages read the other boxes' cells directly gets
-        no same-level copies."""
+        """Ghost cells of level lev's state S at time t; a stage input (stage)
+        of a level whose fused stages read the other boxes' cells directly
+        gets no same-level copies.  Not so the first stage's input of a level
+        with a finer one: it becomes the coarse old state, whose ghost cells
+        the finer level's interpolation reads."""
         L = self.levels[lev]
         key = (lev, id(S))
         if key not in self.direct:
@@ -651,7 +653,7 @@ class Hierarchy:
         A, B, C = self.cur[lev], self.old[lev], self.tmp[lev]
         sin = A
         for s, t in enumerate(times):
-            self._fill(lev, sin, t, stage=True)
+            self._fill(lev, sin, t, stage=s > 0 or lev + 1 == len(self.levels))
             _, mode, a, b, c, d = capi.stage_coeffs(sch.order_rk, sch.stages_rk, dt, s)
             out = B if s % 2 == 0 else C
             L.rk_stage(mode, a, b, c, d, A, sin, out)

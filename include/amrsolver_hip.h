@@ -147,8 +147,9 @@ int amr_fill_two_levels(amr_boxtab_t fine, amr_boxtab_t crse, int ratio, double 
  * kernel reads the cells other boxes hold straight from their arrays
  * (amr_step_plan on that input: info[3] == 3; src/tim/CNS_advance.cpp:54-161
  * fills those ghost cells by copies).  Other stage inputs need
- * amr_fill_two_levels.  On a level with no owner map for such reads it is
- * amr_fill_two_levels.  No reference counterpart. */
+ * amr_fill_two_levels, and so does U^n of a level that a finer one
+ * interpolates from (it is read again as crse_old).  On a level with no owner
+ * map for such reads it is amr_fill_two_levels.  No reference counterpart. */
 int amr_fill_two_levels_cf(amr_boxtab_t fine, amr_boxtab_t crse, int ratio, double a_old,
                            const amr_fab_t* crse_old, double b_new, const amr_fab_t* crse_new, int ngrow,
                            const amr_fab_t* fine_state);

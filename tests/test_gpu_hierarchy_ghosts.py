@@ -62,9 +62,18 @@ def _run(ctx, order, visc, layout):
 
 
 @pytest.mark.parametrize("layout", ["level", "boxes"])
-@pytest.mark.parametrize("order,visc", [(6, True), (6, False)], ids=["keep6v", "keep6"])
+@pytest.mark.parametrize("order,visc", [(6, True), (6, False), (4, True), (2, False)], ids=["keep6v", "keep6", "keep4v", "keep2"])
 def test_hierarchy_matches_the_oracle(ctx, order, visc, layout):
     print(f"case hierarchy ghosts keep{order} visc {visc} {layout}", flush=True)
     for lev, (got, want) in enumerate(zip(_run(ctx, order, visc, layout), _oracle(order, visc))):
         err = rel_err(got, want)
         assert err <= TOL, f"level {lev}: {err:.3e}"
+
+
+@pytest.mark.parametrize("order,visc", [(4, True), (2, False)], ids=["keep4v", "keep2"])
+def test_hierarchy_layouts_agree(ctx, order, visc):
+    """One array per box (whose stages read the other boxes' cells directly)
+    and one array per level: the same bits."""
+    print(f"case hierarchy layouts keep{order} visc {visc}", flush=True)
+    for a, b in zip(_run(ctx, order, visc, "level"), _run(ctx, order, visc, "boxes")):
+        assert np.array_equal(a, b)
