@@ -43,6 +43,7 @@ class Context:
         h = ctypes.c_void_p()
         call("amr_ctx_create", device, ctypes.c_void_p(self.stream.cuda_stream), ctypes.byref(h))
         self.h = h
+        self.choices = 0  # changes of what decides how steps run (tilings, sources)
 
     def synchronize(self):
         call("amr_ctx_synchronize", self.h)
@@ -365,6 +366,7 @@ class Level:
         """Force the fused-kernel tiling for this level's scheme (0,0,0 = auto,
         -1 = pass-structured kernels); form 1 picks the fused kernel's
         self-loading form (16x16 tiles, viscous KEEP 2/4)."""
+        self.ctx.choices += 1
         if form:
             call("amr_set_tiling_form", self.ctx.h, ctypes.byref(self.scheme), tx, ty, tz, form)
         else:
@@ -373,6 +375,7 @@ class Level:
     def set_box_tiling(self, tx, ty, tz):
         """Force the fused-kernel tiling with tiles per box, also on a
         level-wide array."""
+        self.ctx.choices += 1
         call("amr_set_box_tiling", self.ctx.h, ctypes.byref(self.scheme), tx, ty, tz)
 
     def step_plan(self, S):
@@ -389,12 +392,14 @@ class Level:
 
     def autotune(self, S):
         out = (ctypes.c_int32 * 3)()
+        self.ctx.choices += 1
         call("amr_autotune", self.h, ctypes.byref(self.closures), ctypes.byref(self.scheme), S.fabs, out)
         return tuple(out)
 
     def set_source(self, src):
         """Register the source arrays (a StateArrays, or None) added to dSdt
         for schemes with rhs_source = 1."""
+        self.ctx.choices += 1
         call("amr_set_source", self.h, src.fabs if src is not None else None)
 
     def set_user_source(self, code, params=()):
@@ -402,6 +407,7 @@ class Level:
         for this GPU), applied after the flux assembly for schemes with
         rhs_source = 1; None removes it."""
         arr = (ctypes.c_double * max(len(params), 1))(*params)
+        self.ctx.choices += 1
         call("amr_set_user_source", self.h, None if code is None else code.encode(), arr, len(params))
 
     def set_problem(self, wall_T=0.0, body_force_x=0.0, clear=False):
@@ -610,7 +616,9 @@ class Hierarchy:
         self.tmp = [lev.new_state(layout=layout) for lev in self.levels]
         self.tint = [(0.0, 0.0)] * len(self.levels)
         self.ngrow = [None] * len(self.levels)
+        # as step_plan gives them, for the choices in force when they were asked for
         self.direct = {}  # (level, id of a state): its stages read the other boxes' cells directly
+        self.choices = [lev.ctx.choices for lev in self.levels]
 
     def upload(self, us):
         for S, u in zip(self.cur, us):
@@ -627,6 +635,9 @@ class Hierarchy:
         the finer level's interpolation reads."""
         L = self.levels[lev]
         key = (lev, id(S))
+        if self.choices[lev] != L.ctx.choices:
+            self.choices[lev] = L.ctx.choices
+            self.direct = {k: v for k, v in self.direct.items() if k[0] != lev}
         if key not in self.direct:
             # the fused stage kernel reads two ghost layers (three at order 6),
             # the others three; tiles per box may read the other boxes' cells

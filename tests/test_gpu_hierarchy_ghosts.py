@@ -77,3 +77,21 @@ def test_hierarchy_layouts_agree(ctx, order, visc):
     print(f"case hierarchy layouts keep{order} visc {visc}", flush=True)
     for a, b in zip(_run(ctx, order, visc, "level"), _run(ctx, order, visc, "boxes")):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("first,second", [((0,), (-1,)), ((-1,), (0,))], ids=["fused to passes", "passes to fused"])
+def test_tiling_changed_between_steps(ctx, first, second):
+    """The fills follow the kernels that run: the fused stages read the other
+    boxes' cells directly, the pass-structured ones read ghost cells."""
+    from amrsolver_amd import level as L
+    print(f"case hierarchy tiling {first} then {second}", flush=True)
+    sch = P.scheme(flux_euler=1, order_keep=4, visc=True)
+    H = L.Hierarchy([L.Level(g, b, P.closures_reference(), sch, ctx=ctx) for g, b in _levels()], layout="boxes")
+    H.upload(_states())
+    for k, tiling in enumerate((first, second)):
+        H.levels[0].set_tiling(*tiling)  # the scheme's, on every level
+        H.advance(k * DT, DT)
+    H.levels[0].set_tiling(0)
+    for lev, ((_, boxes), want) in enumerate(zip(_levels(), _oracle(4, True))):
+        err = rel_err(_covered(H.download(lev), boxes), want)
+        assert err <= TOL, f"level {lev}: {err:.3e}"
