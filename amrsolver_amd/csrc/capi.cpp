@@ -1546,7 +1546,9 @@ WrapArgs wrap_args(const amr_boxtab_s* bt, DescSet* ds) {
 // directions and bounded in others (a channel).  The self-loading form then
 // reads the periodic images itself, and a stage's fill writes the ghost cells
 // at the physical boundaries only: their sources lie in the same column or
-// row, and the images of the corner ghost cells are read in the domain.
+// row, and the images of the corner ghost cells are read in the domain.  Not
+// beside a boundary of code 0, whose ghost cells the caller keeps: nothing
+// makes those in the corners images of each other.
 bool part_wrap_ok(const amr_boxtab_s* bt, DescSet* ds) {
   if (ds->pwrap >= 0) return ds->pwrap == 1;
   ds->pwrap = 0;
@@ -1556,6 +1558,7 @@ bool part_wrap_ok(const amr_boxtab_s* bt, DescSet* ds) {
   int nper = 0;
   for (int d = 0; d < 3; ++d) {
     nper += g.periodic[d] ? 1 : 0;
+    if (!g.periodic[d] && (g.lo_bc[d] == 0 || g.hi_bc[d] == 0)) return false;
     dom *= g.dom_hi[d] - g.dom_lo[d] + 1;
   }
   if (nper == 0 || nper == 3) return false;
