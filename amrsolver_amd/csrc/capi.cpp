@@ -3512,23 +3512,36 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
   for (auto& B : bt->bt.h_boxes) maxz = std::max(maxz, B.hi[2] - B.lo[2] + 1);
   const int maxz_level = level ? bt->cover.hi[2] - bt->cover.lo[2] + 1 : 0;  // level tiles run across boxes
   std::vector<FusedConfig> cand;
-  const bool self16 = fused_self_supported(*sch, 16, 16) && fused_fits(bt, FusedConfig{16, 16, 16});
   const int shapes[3][2] = {{16, 16}, {32, 8}, {8, 8}};
   // the usual plane counts and the one of least estimated time
   std::vector<int> tzs = {4, 8, 16, 24, 32, 48, 64, 128};
   const int est = default_config(bt, *sch).tz;
   if (std::find(tzs.begin(), tzs.end(), est) == tzs.end()) tzs.push_back(est);
-  for (int box_tiles = level ? 0 : 1; box_tiles <= 1; ++box_tiles)
+  for (int box_tiles = level ? 0 : 1; box_tiles <= 1; ++box_tiles) {
+    // whether 16x16 columns of this kind of tiles run the self-loading form
+    // (tiles over the union also fit boxes that tiles per box leave idle)
+    const bool self16 = fused_self_supported(*sch, 16, 16) && fused_fits(bt, FusedConfig{16, 16, 16}, !box_tiles);
     for (auto& sh : shapes)
       for (int tz : tzs) {
         FusedConfig c{sh[0], sh[1], tz, box_tiles};
         if (tz > 2 * (box_tiles ? maxz : maxz_level) && tz != 16) continue;
-        // short tiles only where longer ones leave the chip idle
-        if (tz < 16 && tz != est && tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz}) >= 1024) continue;
         if (!(fused_supported(*sch, c.tx, c.ty) && fused_fits(bt, c, !box_tiles))) continue;
+        // short tiles only where longer ones leave the chip idle
+        if (tz < 16 && tz != est) {
+          int64_t longer = tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz});
+          if (!box_tiles) {
+            TileTable* tt = nullptr;
+            if ((rc = get_tiles(bt, FusedConfig{c.tx, c.ty, 2 * tz}, true, &tt))) return rc;
+            longer = tt->n;
+          }
+          if (longer >= 1024) continue;
+        }
         // the self-loading form where there is one (TGV 256^3, KEEP4: 0.67
-        // ms a stage against 0.77; KEEP2 0.59 against 0.64), which also
-        // leaves 32x8 columns behind (1.2 ms); next to walls only that form
+        // ms a stage against 0.77; KEEP2 0.59 against 0.64; 96^3 refined in
+        // boxes of 8 held as one array 107 us a step against 117), which also
+        // leaves 32x8 columns behind (1.2 ms; boxes 32x8x32, whose 16x16
+        // columns are half idle, 254 us a step with them, 250 without); next
+        // to walls only that form
         if (self16) {
           if (!fused_self_supported(*sch, c.tx, c.ty) && (c.tx != 8 || bt->wall_args.nkeep_blk > 0)) continue;
           c.form = c.tx == 16 ? 1 : 0;
@@ -3537,6 +3550,7 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
         }
         cand.push_back(c);
       }
+  }
   if (cand.empty()) {
     bt->tuned[key] = FusedConfig{-1, 0, 0};
     tiling[0] = -1;
