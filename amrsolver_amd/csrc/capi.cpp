@@ -1020,10 +1020,42 @@ bool cover_bit(const amr_boxtab_s* bt, int64_t bx, int64_t by, int64_t bz) {
   return (bt->cover_bits[size_t(bit >> 5)] >> (bit & 31)) & 1u;
 }
 
-// Tiles of the fused kernel: box by box, or (level tiling) TX x TY columns on
-// a grid anchored at the bounding box's corner, split into runs of planes
-// that hold covered cells, each run cut into near-equal pieces of at most
-// tz planes.
+// Level tiling: TX x TY columns on a grid anchored at the bounding box's
+// corner, split into runs of planes that hold covered cells (tiles of whole
+// runs).
+std::vector<TileDev> level_runs(const amr_boxtab_s* bt, int tx, int ty) {
+  std::vector<TileDev> out;
+  const Cover& c = bt->cover;
+  const int sh = c.sh;
+  for (int j0 = c.lo[1]; j0 <= c.hi[1]; j0 += ty)
+    for (int i0 = c.lo[0]; i0 <= c.hi[0]; i0 += tx) {
+      const int bx0 = (i0 - c.lo[0]) >> sh, bx1 = std::min(i0 + tx - 1 - c.lo[0], c.hi[0] - c.lo[0]) >> sh;
+      const int by0 = (j0 - c.lo[1]) >> sh, by1 = std::min(j0 + ty - 1 - c.lo[1], c.hi[1] - c.lo[1]) >> sh;
+      auto plane_block_used = [&](int bz) {
+        for (int by = by0; by <= by1; ++by)
+          for (int bx = bx0; bx <= bx1; ++bx)
+            if (cover_bit(bt, bx, by, bz)) return true;
+        return false;
+      };
+      int bz = 0;
+      while (bz < c.nb[2]) {
+        if (!plane_block_used(bz)) {
+          ++bz;
+          continue;
+        }
+        int ez = bz;
+        while (ez + 1 < c.nb[2] && plane_block_used(ez + 1)) ++ez;
+        const int k0 = c.lo[2] + (bz << sh);
+        const int k1 = std::min(c.hi[2], c.lo[2] + ((ez + 1) << sh) - 1);
+        out.push_back(TileDev{0, i0, j0, k0, k1 - k0 + 1});
+        bz = ez + 1;
+      }
+    }
+  return out;
+}
+
+// Tiles of the fused kernel: box by box, or (level tiling) the runs of
+// level_runs, each cut into near-equal pieces of at most tz planes.
 int get_tiles(amr_boxtab_s* bt, const FusedConfig& cfg, bool level, TileTable** out) {
   auto key = std::make_tuple(cfg.tx, cfg.ty, cfg.tz, level ? 1 : 0);
   auto it = bt->tiles.find(key);
@@ -1033,39 +1065,15 @@ int get_tiles(amr_boxtab_s* bt, const FusedConfig& cfg, bool level, TileTable** 
   }
   std::vector<TileDev> logical;
   if (level) {
-    const Cover& c = bt->cover;
-    const int sh = c.sh;
-    for (int j0 = c.lo[1]; j0 <= c.hi[1]; j0 += cfg.ty)
-      for (int i0 = c.lo[0]; i0 <= c.hi[0]; i0 += cfg.tx) {
-        const int bx0 = (i0 - c.lo[0]) >> sh, bx1 = std::min(i0 + cfg.tx - 1 - c.lo[0], c.hi[0] - c.lo[0]) >> sh;
-        const int by0 = (j0 - c.lo[1]) >> sh, by1 = std::min(j0 + cfg.ty - 1 - c.lo[1], c.hi[1] - c.lo[1]) >> sh;
-        auto plane_block_used = [&](int bz) {
-          for (int by = by0; by <= by1; ++by)
-            for (int bx = bx0; bx <= bx1; ++bx)
-              if (cover_bit(bt, bx, by, bz)) return true;
-          return false;
-        };
-        int bz = 0;
-        while (bz < c.nb[2]) {
-          if (!plane_block_used(bz)) {
-            ++bz;
-            continue;
-          }
-          int ez = bz;
-          while (ez + 1 < c.nb[2] && plane_block_used(ez + 1)) ++ez;
-          const int k0 = c.lo[2] + (bz << sh);
-          const int k1 = std::min(c.hi[2], c.lo[2] + ((ez + 1) << sh) - 1);
-          const int run = k1 - k0 + 1;
-          const int pieces = (run + cfg.tz - 1) / cfg.tz;
-          int k = k0;
-          for (int p = 0; p < pieces; ++p) {
-            const int nz = run / pieces + (p < run % pieces ? 1 : 0);
-            logical.push_back(TileDev{0, i0, j0, k, nz});
-            k += nz;
-          }
-          bz = ez + 1;
-        }
+    for (const TileDev& r : level_runs(bt, cfg.tx, cfg.ty)) {
+      const int pieces = (r.nz + cfg.tz - 1) / cfg.tz;
+      int k = r.k0;
+      for (int p = 0; p < pieces; ++p) {
+        const int nz = r.nz / pieces + (p < r.nz % pieces ? 1 : 0);
+        logical.push_back(TileDev{0, r.i0, r.j0, k, nz});
+        k += nz;
       }
+    }
   } else {
     for (int b = 0; b < bt->bt.nbox; ++b) {
       const BoxDev& B = bt->bt.h_boxes[b];
@@ -1151,36 +1159,69 @@ bool fused_fits(const amr_boxtab_s* bt, const FusedConfig& cfg, bool level = fal
   return 2 * cells_ >= lanes;
 }
 
-// Tiles per box of a tiling, and its estimated time: a tile costs a plane
-// iteration per plane plus three for the pipeline; `slots` workgroups fit the
-// chip at once (the 16x16 kernels two per CU, KEEP6 one, 8x8 columns eight),
-// and an iteration takes 1.35 times as long once the CUs are shared (128x64x64
-// viscous KEEP4, self-loading form: 64 tiles of 32 planes 3.6 us an
-// iteration, 512 tiles of 4 planes 5.0 us).
-int64_t tile_count(const amr_boxtab_s* bt, const FusedConfig& cfg, int64_t* iters = nullptr, int* longest = nullptr) {
+// Workgroups of a fused stage kernel that a CU holds.  16x16 columns: two
+// (LDS, or two waves per SIMD), order 6 one (one wave per SIMD).  8x8 columns,
+// a wave each: eight (two waves per SIMD), viscous six (25 KB of LDS each),
+// order 6 four (again one wave per SIMD).  A round too many costs as much as
+// the one before it: 64^3 in boxes of 8, one array, KEEP4 viscous 82 us a step
+// with three planes a tile (1536 tiles, six a CU), 120 with two (2048); order 6
+// 125 with four planes (1024 tiles), 172 with three.
+int tiles_per_cu(const amr_scheme_t& sch, const FusedConfig& cfg) {
+  if (cfg.tx * cfg.ty != 64) return sch.order_keep == 6 ? 1 : 2;
+  return sch.order_keep == 6 ? 4 : (sch.rhs_visc ? 6 : 8);
+}
+
+// Columns of a tiling by their planes: tiles per box, or over the union.
+struct Columns {
+  int planes;
+  int64_t count;
+};
+std::vector<Columns> tile_columns(const amr_boxtab_s* bt, int tx, int ty, bool level) {
+  std::vector<Columns> out;
+  if (level) {
+    for (const TileDev& r : level_runs(bt, tx, ty)) out.push_back({r.nz, 1});
+  } else {
+    for (auto& B : bt->bt.h_boxes)
+      out.push_back({B.hi[2] - B.lo[2] + 1,
+                     int64_t((B.hi[0] - B.lo[0] + tx) / tx) * ((B.hi[1] - B.lo[1] + ty) / ty)});
+  }
+  return out;
+}
+
+// Tiles of those columns, their plane iterations (a tile costs one per plane
+// plus three for the pipeline) and the longest tile's.
+int64_t tile_count(const std::vector<Columns>& cols, int tz, int64_t* iters = nullptr, int* longest = nullptr) {
   int64_t n = 0, it = 0;
   int mx = 0;
-  for (auto& B : bt->bt.h_boxes) {
-    const int64_t cols = int64_t((B.hi[0] - B.lo[0] + cfg.tx) / cfg.tx) * ((B.hi[1] - B.lo[1] + cfg.ty) / cfg.ty);
-    const int nz = B.hi[2] - B.lo[2] + 1, full = nz / cfg.tz, rem = nz % cfg.tz;
-    n += cols * (full + (rem ? 1 : 0));
-    it += cols * (int64_t(full) * (cfg.tz + 3) + (rem ? rem + 3 : 0));
-    mx = std::max(mx, std::min(nz, cfg.tz) + 3);
+  for (const Columns& c : cols) {
+    const int pieces = (c.planes + tz - 1) / tz;
+    n += c.count * pieces;
+    it += c.count * (c.planes + 3 * int64_t(pieces));
+    mx = std::max(mx, std::min(c.planes, tz) + 3);
   }
   if (iters) *iters = it;
   if (longest) *longest = mx;
   return n;
 }
 
-double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedConfig& cfg) {
+// Estimated time of a tiling.  An iteration takes longer once SIMDs hold more
+// than one wave, which order 6 never does: 1.35 times (128x64x64 viscous KEEP4,
+// self-loading form: 64 tiles of 32 planes 3.6 us an iteration, 512 tiles of 4
+// planes 5.0 us).  Six waves a CU are two on some SIMDs and one on others: one
+// round takes as long as the former, 1.2 to 1.3 times, several average out
+// (100^3 in boxes of 20, KEEP4 viscous, one array: 1125 tiles of 20 planes 404
+// us a step, 3375 of 6 and 7 planes 381, 4500 of 5 planes 359; 40^3: 720 tiles
+// of two planes 58, 1440 of one 57).
+double tiling_time(const std::vector<Columns>& cols, const amr_scheme_t& sch, const FusedConfig& cfg) {
   int64_t it = 0;
   int mx = 0;
-  const int64_t n = tile_count(bt, cfg, &it, &mx);
-  const int64_t slots = 256 * (cfg.tx * cfg.ty == 64 ? 8 : (sch.order_keep == 6 ? 1 : 2));
-  if (n <= std::max<int64_t>(256, slots / 2)) return mx;
+  const int64_t n = tile_count(cols, cfg.tz, &it, &mx);
+  const int64_t slots = 256 * tiles_per_cu(sch, cfg), alone = 256 * (256 / (cfg.tx * cfg.ty));
+  if (n <= alone) return mx;
+  const double shared = slots <= alone ? 1.0 : (slots % alone == 0 ? 1.35 : (n <= slots ? 1.24 : 1.08));
   // whole rounds of the longest tiles while there are few, an even load later
   const double rounds = n <= 4 * slots ? double((n + slots - 1) / slots) * mx : double(it) / slots;
-  return 1.35 * std::max(rounds, double(mx));
+  return shared * std::max(rounds, double(mx));
 }
 
 // Plane counts of tiles that the estimates choose from: dense where tiles are
@@ -1189,8 +1230,9 @@ double tiling_time(const amr_boxtab_s* bt, const amr_scheme_t& sch, const FusedC
 // slots empty, 7 fill them).
 constexpr int TILE_PLANES[] = {64, 48, 32, 24, 20, 16, 14, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2, 1};
 
-std::array<int, 6> estimate_key(const amr_scheme_t& s, int reverse) {
-  return {s.rhs_euler, s.rhs_visc, s.flux_euler, s.order_keep, s.art_diss, reverse};
+// kind 0: forward, tiles per box; 1: reverse; 2: forward, over the union
+std::array<int, 6> estimate_key(const amr_scheme_t& s, int kind) {
+  return {s.rhs_euler, s.rhs_visc, s.flux_euler, s.order_keep, s.art_diss, kind};
 }
 
 // The tiling of a table that has not been autotuned: 16x16 columns (in the
@@ -1198,39 +1240,43 @@ std::array<int, 6> estimate_key(const amr_scheme_t& s, int reverse) {
 // with the plane count of least estimated time -- short tiles where a level
 // has too few columns to fill the chip (32x24x20 in 8 boxes: 8x8x64 took
 // 90 us a right-hand side, 16x16x4 takes 26, 16x16x1 14; order 6 on 40x47x33,
-// the CFL estimate included, 261, 70, 51).
-FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
-  const auto known = bt->estimated.find(estimate_key(sch, 0));
+// the CFL estimate included, 261, 70, 51).  The columns are those of the kind
+// of tiles asked for; their shape is the tiles per box's.
+FusedConfig default_config(const amr_boxtab_s* bt, const amr_scheme_t& sch, bool level) {
+  level = level && bt->cover.on;
+  const auto key = estimate_key(sch, level ? 2 : 0);
+  const auto known = bt->estimated.find(key);
   if (known != bt->estimated.end()) return known->second;
   FusedConfig c{16, 16, 64};
   if (fused_self_supported(sch, 16, 16)) c.form = 1;
   if (!fused_fits(bt, c)) c = FusedConfig{8, 8, 64};
+  const std::vector<Columns> cols = tile_columns(bt, c.tx, c.ty, level);
   double best = 0.0;
   FusedConfig out = c;
   for (int tz : TILE_PLANES) {
     c.tz = tz;
-    const double t = tiling_time(bt, sch, c);
+    const double t = tiling_time(cols, sch, c);
     if (tz == 64 || t < best) {
       best = t;
       out = c;
     }
   }
-  bt->estimated[estimate_key(sch, 0)] = out;
+  bt->estimated[key] = out;
   return out;
 }
 
-FusedConfig choose_config(const amr_boxtab_s* bt, const amr_scheme_t& sch) {
+FusedConfig choose_config(const amr_boxtab_s* bt, const amr_scheme_t& sch, bool level = false) {
   const std::string key = scheme_key(sch);
   auto tk = bt->ctx->tuned.find(key);
   if (tk != bt->ctx->tuned.end()) return tk->second;
   auto tb = bt->tuned.find(key);
   if (tb != bt->tuned.end()) return tb->second;
-  return default_config(bt, sch);
+  return default_config(bt, sch, level);
 }
 
 // Whether the fused stage kernel handles this scheme on this table.
 bool fused_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, FusedConfig* out, bool level = false) {
-  FusedConfig cfg = choose_config(bt, sch);
+  FusedConfig cfg = choose_config(bt, sch, level);
   if (out) *out = cfg;
   // fluxes next to walls: the self-loading form (WallRows), else the
   // pass-structured kernels' corrections
@@ -1961,7 +2007,7 @@ int prepare_step_tables(amr_boxtab_s* bt, const amr_scheme_t& sch, const amr_fab
                      (bt->wall_args.nkeep_blk == 0 || cfg.form == 1) && !(sch.rhs_source && bt->usrc_fn);
   TileTable* tt = nullptr;
   if (fused && fused_fits(bt, cfg) && (rc = get_tiles(bt, cfg, false, &tt))) return rc;
-  if (fused && bt->cover.on && (rc = get_tiles(bt, cfg, true, &tt))) return rc;
+  if (fused && bt->cover.on && (rc = get_tiles(bt, choose_config(bt, sch, true), true, &tt))) return rc;
   bool tube = false;
   if (!(fused && fused_fits(bt, cfg)) && ((rc = tube_path(bt, sch, &tube)) || (!tube && (rc = ensure_unfused(bt, sch)))))
     return rc;
@@ -2192,12 +2238,13 @@ bool march_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, const StageArgs
     return true;
   }
   const int64_t slots = 256 * adj_march_per_cu(sch);
+  const std::vector<Columns> cols = tile_columns(bt, cfg.tx, cfg.ty, false);
   double best = 0.0;
   for (int tz : TILE_PLANES) {
     cfg.tz = tz;
     int64_t it = 0;
     int mx = 0;
-    const int64_t n = tile_count(bt, cfg, &it, &mx);  // three iterations more than planes per tile
+    const int64_t n = tile_count(cols, tz, &it, &mx);  // three iterations more than planes per tile
     double t = mx - 1;
     if (n > 256) t = 1.35 * std::max(t, n <= 4 * slots ? double((n + slots - 1) / slots) * t : double(it - n) / slots);
     if (tz == 64 || t < best) {
@@ -3513,29 +3560,22 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
   const int maxz_level = level ? bt->cover.hi[2] - bt->cover.lo[2] + 1 : 0;  // level tiles run across boxes
   std::vector<FusedConfig> cand;
   const int shapes[3][2] = {{16, 16}, {32, 8}, {8, 8}};
-  // the usual plane counts and the one of least estimated time
-  std::vector<int> tzs = {4, 8, 16, 24, 32, 48, 64, 128};
-  const int est = default_config(bt, *sch).tz;
-  if (std::find(tzs.begin(), tzs.end(), est) == tzs.end()) tzs.push_back(est);
   for (int box_tiles = level ? 0 : 1; box_tiles <= 1; ++box_tiles) {
     // whether 16x16 columns of this kind of tiles run the self-loading form
     // (tiles over the union also fit boxes that tiles per box leave idle)
     const bool self16 = fused_self_supported(*sch, 16, 16) && fused_fits(bt, FusedConfig{16, 16, 16}, !box_tiles);
-    for (auto& sh : shapes)
+    // the usual plane counts and the one of least estimated time
+    std::vector<int> tzs = {4, 8, 16, 24, 32, 48, 64, 128};
+    const int est = default_config(bt, *sch, !box_tiles).tz;
+    if (std::find(tzs.begin(), tzs.end(), est) == tzs.end()) tzs.push_back(est);
+    for (auto& sh : shapes) {
+      const std::vector<Columns> cols = tile_columns(bt, sh[0], sh[1], !box_tiles);
       for (int tz : tzs) {
         FusedConfig c{sh[0], sh[1], tz, box_tiles};
         if (tz > 2 * (box_tiles ? maxz : maxz_level) && tz != 16) continue;
         if (!(fused_supported(*sch, c.tx, c.ty) && fused_fits(bt, c, !box_tiles))) continue;
         // short tiles only where longer ones leave the chip idle
-        if (tz < 16 && tz != est) {
-          int64_t longer = tile_count(bt, FusedConfig{c.tx, c.ty, 2 * tz});
-          if (!box_tiles) {
-            TileTable* tt = nullptr;
-            if ((rc = get_tiles(bt, FusedConfig{c.tx, c.ty, 2 * tz}, true, &tt))) return rc;
-            longer = tt->n;
-          }
-          if (longer >= 1024) continue;
-        }
+        if (tz < 16 && tz != est && tile_count(cols, 2 * tz) >= 1024) continue;
         // the self-loading form where there is one (TGV 256^3, KEEP4: 0.67
         // ms a stage against 0.77; KEEP2 0.59 against 0.64; 96^3 refined in
         // boxes of 8 held as one array 107 us a step against 117), which also
@@ -3550,6 +3590,7 @@ int amr_autotune(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t*
         }
         cand.push_back(c);
       }
+    }
   }
   if (cand.empty()) {
     bt->tuned[key] = FusedConfig{-1, 0, 0};
