@@ -180,17 +180,21 @@ __device__ __forceinline__ double weno5js(double s0, double s1, double s2, doubl
   return (1.0 / 6.0) * sum * (a0 * v0 + a1 * v1 + a2 * v2);
 }
 
-// weno5js with fewer operations and the same rounding.  It is bound by FP64
-// issue and its four divisions are half of that when each expands by itself
-// (13 instructions' time each), so the three weights share one reciprocal of
-// the product of their denominators, refined as a division's is, and each
-// quotient takes the division's own last step (residual by fma, one
-// correction); 2x, 4x and x/4 are exact, so fma with them rounds as the
-// separate operations do.  Holds where the product of the denominators is a
-// normal number; elsewhere (a smoothness sum of 1e49 or more, or NaN) `ok` is
-// cleared and the result is not to be used.  The batch of 512 1D problems
-// (8.65M cells) went from 1.41 to 1.24 ms a stage, viscous WENO on 100x96x92
-// from 410 to 363 us.
+// weno5js with fewer operations.  It is bound by FP64 issue and its four
+// divisions are half of that when each expands by itself (13 instructions' time
+// each), so the three weights share one reciprocal of the product of their
+// denominators, refined as a division's is, and each quotient takes the
+// division's own last step (residual by fma, one correction); 2x, 4x and x/4
+// are exact, so fma with them rounds as the separate operations do.  The
+// quotients round as divisions do except within a few 2^-53 ulp of a tie (the
+// reciprocal of one denominator is a product, good to a few ulps); none of the
+// 1e7 compared did.  Holds where the product of the denominators stays below
+// 1e304, that is for differences of up to some 1e18 (the centre sum is a fourth
+// power); a single reciprocal that is not a normal number then belongs to a
+// denominator 1e140 times another one, whose weight does not enter.  Elsewhere,
+// or for NaN, `ok` is cleared and the result is not to be used.  The batch of
+// 512 1D problems (8.65M cells) went from 1.41 to 1.24 ms a stage, viscous WENO
+// on 100x96x92 from 410 to 363 us.
 __device__ __forceinline__ double weno5js_fast(double s0, double s1, double s2, double s3, double s4, bool& ok) {
   const double eps = 1e-40;
   const double m3 = 3.0 * s2;
@@ -201,9 +205,10 @@ __device__ __forceinline__ double weno5js_fast(double s0, double s1, double s2, 
   const double b1 = __builtin_fma(0.25, e1 * e1 * e1 * e1, (13.0 / 12.0) * c1 * c1);
   const double b2 = __builtin_fma(0.25, e2 * e2, (13.0 / 12.0) * c2 * c2);
   const double t0 = eps + b0, t1 = eps + b1, t2 = eps + b2;
-  ok = ok && t0 + t1 + t2 < 1e49;
   const double d0 = t0 * t0, d1 = t1 * t1, d2 = t2 * t2;
-  const double d12 = d1 * d2, r = rcp_refined(d0 * d12), rd0 = r * d0;
+  const double d12 = d1 * d2, d = d0 * d12;
+  ok = ok && d < 1e304;
+  const double r = rcp_refined(d), rd0 = r * d0;
   const double a0 = div_by_rcp(0.1, d0, r * d12);
   const double a1 = div_by_rcp(0.6, d1, rd0 * d2);
   const double a2 = div_by_rcp(0.3, d2, rd0 * d1);
