@@ -856,9 +856,9 @@ int copy_uncovered(amr_boxtab_s* bt, const DescSet* from, const DescSet* to, con
 enum { UW_PRIMS = 1, UW_VISC = 2, UW_WENO = 4, UW_SLOPE = 8, UW_JST = 16 };
 
 // Brick table of the tube stages: side tables (so every box spans its
-// periodic y and z extents) and boxes 4 x 4 cells across.  Split bricks while
-// they fill less than a few rounds of the chip (one workgroup a CU): above
-// that the long bricks' throughput wins.
+// periodic y and z extents) and boxes 4 x 4 cells across.  Split bricks up to
+// two rounds of the chip (a CU holds one WENO workgroup of 15 waves): above
+// that the long bricks are faster (the times stand beside TUBE_SPLIT_MAX).
 int build_tube(amr_boxtab_s* bt) {
   if (bt->tube_built) return AMR_OK;
   bool is = bt->d_xside != nullptr;
@@ -2226,9 +2226,14 @@ int ensure_adjoint_level(amr_boxtab_s* bt, const amr_scheme_t& s) {
 // its tiles: KEEP order 2/4, boxes that fill most lanes of 16x16 columns (the
 // passes gather a cell per lane of any box), and the plane count of least
 // estimated time.  A tile costs an iteration per plane plus two, 1.35 times as
-// long once CUs are shared.  Measured, 8 steps checkpointed every 3, tz 1, 2,
-// 4, 8 (passes): 24^3 976, 1076, 1342, 1896 us (1171); 96x48x40 1362, 1345,
-// 1489, 2063 (1845); 126x71x72 3768, 3401, 3304, 3288, tz 6 3084 (5728).
+// long once CUs are shared.  Measured for every plane count on eleven tables
+// from 24^3 to 160^3, viscous order 4 and inviscid order 2: the choice is within
+// 12% of the best.  A reverse stage, us, estimated choice (best): 24^3 13.2 (1
+// plane), 48^3 20.6, 2 planes (18.8, 1), 128x64x64 52.8, 4 (4), 96^3 76, 7 (7),
+// 130x126x64 106, 11 (11), 200x180x37 149, 14 (133, 7), 160^3 349, 32 (32);
+// inviscid order 2, three workgroups a CU: 128x64x64 42.2, 3 (38.7, 4),
+// 126x71x72 61.6 (55.4, 6).  Passes, 8 steps checkpointed every 3: 24^3 1171 us
+// (976), 96x48x40 1845 (1362), 126x71x72 5728 (3084).
 bool march_path(const amr_boxtab_s* bt, const amr_scheme_t& sch, const StageArgs& sa, FusedConfig* out) {
   FusedConfig cfg{16, 16, 64};
   if (!adj_march_supported(sch) || sa.box_dt || !fused_fits(bt, cfg)) return false;

@@ -187,8 +187,8 @@ __device__ __forceinline__ double weno5js(double s0, double s1, double s2, doubl
 // division's own last step (residual by fma, one correction); 2x, 4x and x/4
 // are exact, so fma with them rounds as the separate operations do.  The
 // quotients round as divisions do except within a few 2^-53 ulp of a tie (the
-// reciprocal of one denominator is a product, good to a few ulps); none of the
-// 1e7 compared did.  Holds where the product of the denominators stays below
+// reciprocal of one denominator is a product, good to a few ulps); none of
+// the 8e6 compared did.  Holds where the product of the denominators stays below
 // 1e304, that is for differences of up to some 1e18 (the centre sum is a fourth
 // power); a single reciprocal that is not a normal number then belongs to a
 // denominator 1e140 times another one, whose weight does not enter.  Elsewhere,

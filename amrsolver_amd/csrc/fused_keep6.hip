@@ -306,7 +306,7 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
         for (int n = 0; n < 5; ++n) fz_prev[n] = fz[n];
       }
       if (p == k0 + nz + 2) break;  // uniform: that was the tile's last face
-        double s[5];
+      double s[5];
       pair_terms<2>(o, Cell{q2[QRHO], q2[QU], q2[QV], q2[QW], q2[QT], q2[QPRES]}, cv, co1, s);
 #pragma unroll
       for (int n = 0; n < 5; ++n) {
@@ -314,7 +314,7 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
         fb[n] = s[n];
         q1t[n] = t[n];
       }
-        pair_terms<2>(o, lds_cell(s_q, own), cv, co0, s);
+      pair_terms<2>(o, lds_cell(s_q, own), cv, co0, s);
 #pragma unroll
       for (int n = 0; n < 5; ++n) fb[n] = s[n] + fb[n];
     }
@@ -364,18 +364,18 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
       const Cell o = lds_cell(s_q, own);
       double t[5];
       pair_terms<1>(o, lds_cell(s_q, own - RX), cv, co0, ay);
-        pair_terms<1>(o, lds_cell(s_q, own - 2 * RX), cv, co1, t);
+      pair_terms<1>(o, lds_cell(s_q, own - 2 * RX), cv, co1, t);
 #pragma unroll
       for (int n = 0; n < 5; ++n) s_e[n][E_P + tid] = t[n];
-        pair_terms<1>(o, lds_cell(s_q, own - 3 * RX), cv, co2, t);
+      pair_terms<1>(o, lds_cell(s_q, own - 3 * RX), cv, co2, t);
 #pragma unroll
       for (int n = 0; n < 5; ++n) s_e[n][E_Q + tid] = t[n];
-        pair_terms<0>(o, lds_cell(s_q, own - 1), cv, co0, fx);
-        pair_terms<0>(o, lds_cell(s_q, own - 2), cv, co1, px);
+      pair_terms<0>(o, lds_cell(s_q, own - 1), cv, co0, fx);
+      pair_terms<0>(o, lds_cell(s_q, own - 2), cv, co1, px);
 #pragma unroll
       for (int n = 0; n < 5; ++n) fx[n] += px[n];
-        pair_terms<0>(o, lds_cell(s_q, own - 3), cv, co2, qx);
-        if (!ring) {
+      pair_terms<0>(o, lds_cell(s_q, own - 3), cv, co2, qx);
+      if (!ring) {
         // pairs of the cells past the tile
         const Cell a = lds_cell(s_q, eidx), b = lds_cell(s_q, eidx - edist * estr);
         keep_terms_xy(ex_, a.rho, a.u, a.v, a.w, cv * a.T, a.p, b.rho, b.u, b.v, b.w, cv * b.T, b.p, t);

@@ -65,6 +65,11 @@ struct WenoWork {
 struct TubeBrick {
   int box, x0, nx, wrap;
 };
+// Split up to TUBE_SPLIT_MAX short bricks, one line for both fluxes since a
+// table serves both.  Measured, us a stage, short bricks / long ones, tubes of
+// 86, 256, 427, 512, 600, 768 and 1024 short bricks: WENO 6.5/11.7, 9.9/11.9,
+// 11.1/12.2, 13.7/12.1, 15.3/12.2, 15.8/12.4, 22.1/13.0; MUSCL 8.8/12.3,
+// 10.5/12.4, 11.9/12.8, 12.1/12.7, 12.9/12.9, 13.4/13.1, 16.9/13.7.
 constexpr int TUBE_NX = 15, TUBE_SPLIT_NX = 3, TUBE_SPLIT_MAX = 512;
 struct TubeWork {
   TubeBrick* d = nullptr;

@@ -32,9 +32,9 @@ __global__ void __launch_bounds__(BLK) k_prims(const BoxDev* boxes, const BlockR
 
 // ---------------------------------------------------------------- KEEP
 // CentralKEEP.h:40-145 on grownnodaltilebox(-1,0).  Order 4 is held to four
-// waves a SIMD: it is bound by its gathered values (12 a pair), and
-// a fifth wave (96 registers instead of 98) costs more L1 than it hides
-// (96^3: 57.1 us with four, 60.4 with five).
+// waves a SIMD: the fifth, which fits where the compiler takes 96 registers
+// instead of 98, makes it slower (96^3: 57.1 us with four, 60.4 with five).
+// What bounds it is the gather of its neighbours' values through L1.
 template <int H>
 __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(H == 2 ? 4 : 1, H == 2 ? 4 : 8)))
 k_keep(const BoxDev* boxes, const BlockRef* bmap, Region reg, const double* box_dt, const Fab* pr,

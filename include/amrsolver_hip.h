@@ -284,7 +284,9 @@ int amr_stage_coeffs(int order_rk, int stages_rk, double dt, int stage, int* nst
  * = per stage FillPatch + compute_rhs + stage update.  `state` (ng >= 3)
  * holds U^n on entry and U^{n+1} on exit (valid cells; ghost cells are not
  * guaranteed to be filled on exit: a periodic level held as one array is
- * advanced without ghost fills, its halos read from periodic images).  Uses
+ * advanced without ghost fills, its halos read from periodic images; a bounded
+ * one that fills its domain may fill the ghost cells at the physical boundaries
+ * only, and stages that read the other boxes' arrays none of those).  Uses
  * two ghosted workspace arrays owned by the box table. */
 int amr_advance(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme_t* sch,
                 const amr_fab_t* state, double time, double dt);
