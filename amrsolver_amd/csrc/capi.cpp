@@ -1469,6 +1469,17 @@ int build_srcmap(amr_boxtab_s* bt) {
   if (!bt->cover.on || bt->nuncov_cells == 0) return AMR_OK;
   const Cover& c = bt->cover;
   const amr_geom_t& g = bt->geom;
+  // a boundary's fill takes its values from the stage input: where those are
+  // uncovered ghost cells (of the same box, at most NGHOST cells from the
+  // boundary), the input has to hold them
+  int64_t nun = 0;
+  for (const CopyTask& t : uncovered_pieces(bt, NGHOST, &nun)) {
+    const BoxDev& B = bt->bt.h_boxes[t.dst];
+    for (int d = 0; d < 3; ++d)
+      if (!g.periodic[d] && ((B.lo[d] - NGHOST < g.dom_lo[d] && t.lo[d] < g.dom_lo[d] + NGHOST) ||
+                             (B.hi[d] + NGHOST > g.dom_hi[d] && t.hi[d] > g.dom_hi[d] - NGHOST)))
+        return AMR_OK;
+  }
   int sh = c.sh;
   auto aligned = [&](int sh_) {
     for (int d = 0; d < 3; ++d)
