@@ -158,6 +158,7 @@ struct DescSet {
   int wrap = -1;   // one array over the whole periodic domain (-1 unknown)
   int pwrap = -1;  // one array over a whole domain periodic in some directions only (-1 unknown)
   int level = -1;  // one array holding the boxes' bounding box (-1 unknown)
+  int below = 0, above = 0, edge = 0;  // then: as in Cover
   // fill tasks of the inner 1 or 2 ghost layers only (the fused stage
   // kernel reads two); their Fab table is this set's `d`
   std::unique_ptr<DescSet> narrow[2];
@@ -1534,7 +1535,8 @@ int build_srcmap(amr_boxtab_s* bt) {
 
 // Every box of `ds` is a window of one array (same mapping) whose address
 // range also holds what level tiles touch: the boxes' bounding box grown by
-// NGHOST in x and y and by two planes in z.  The address range of an array
+// NGHOST in x and y and by two planes in z (order 6 loads three, of the third
+// what the windows hold).  The address range of an array
 // is taken as the span of its boxes' windows (first to last element), all
 // of which lie in the caller's allocation.
 bool level_ok(const amr_boxtab_s* bt, DescSet* ds) {
@@ -1559,6 +1561,12 @@ bool level_ok(const amr_boxtab_s* bt, DescSet* ds) {
   const intptr_t a1 = m0.origin + 8 * intptr_t((c.hi[0] + NGHOST) + (c.hi[1] + NGHOST) * m0.js +
                                                (c.hi[2] + 2) * m0.ks + (NCONS - 1) * m0.ns) + 8;
   if (a0 < lo || a1 > hi) return false;
+  const int64_t first = (lo - m0.origin) / 8 - (c.lo[2] - 3) * m0.ks;
+  const int64_t last = (hi - m0.origin) / 8 - 1 - (NCONS - 1) * m0.ns - (c.hi[2] + 3) * m0.ks;
+  ds->below = int(std::max<int64_t>(first, INT_MIN));
+  ds->above = int(std::min<int64_t>(last, INT_MAX));
+  ds->edge = first > (c.lo[0] - NGHOST) + (c.lo[1] - NGHOST) * m0.js ||
+             last < (c.hi[0] + NGHOST) + (c.hi[1] + NGHOST) * m0.js;
   ds->level = 1;
   return true;
 }
@@ -1644,7 +1652,7 @@ WrapArgs part_wrap_args(const amr_boxtab_s* bt) {
 // The fused kernel's view of the coverage: the level's bitmap under level
 // tiling, else (and for a fully covered level) one all-ones word that every
 // cell maps to (block edge 2^30).
-Cover kernel_cover(const amr_boxtab_s* bt, bool level) {
+Cover kernel_cover(const amr_boxtab_s* bt, bool level, const DescSet* sin) {
   Cover c{};
   if (level) c = bt->cover;
   c.on = level ? 1 : 0;
@@ -1653,6 +1661,9 @@ Cover kernel_cover(const amr_boxtab_s* bt, bool level) {
     c.sh = 30;
     for (int d = 0; d < 3; ++d) c.nb[d] = 1;
   }
+  c.below = level ? sin->below : INT_MIN;
+  c.above = level ? sin->above : INT_MAX;
+  c.edge = level ? sin->edge : 0;
   return c;
 }
 
@@ -1799,7 +1810,7 @@ int do_stage(amr_boxtab_s* bt, const amr_closures_t& cls, const amr_scheme_t& sc
       us = bt->srcmap;
       us.u0 = uncov_u0;
     }
-    const Cover cov = kernel_cover(bt, level);
+    const Cover cov = kernel_cover(bt, level, dsin);
     NbMap nbm = !uncov_u0 && nb_direct(bt, sch, level, dsin) ? bt->nbmap : NbMap{};
     nbm.ustride = nbm.on && dsin->ustride == 1 ? 1 : 0;
     WallRows wr{};

@@ -75,7 +75,11 @@ struct Cfg {
 // reads of equal strides, which fits 168 registers without a spill only when
 // asked to (left at two it took 174: 128x100x100 in boxes of 64x20x10 224 us
 // a step, at three 210; with a source it spills at three).
-template <int H, bool VISC, int TX, int TY, bool UCS, bool SRC, int NB>
+// EDGE: level tiles of order 6 whose array is not known to hold every cell of the
+// planes three from the bounding box (Cover::below, above; compiled for its own:
+// the bounds cost tiles of one plane 2 to 4%, 32^3 in boxes of 8^3 58 -> 60 us a
+// step).
+template <int H, bool VISC, int TX, int TY, bool UCS, bool SRC, int NB, bool EDGE>
 __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H == 3 ? 1 : (H == 1 && !VISC && TX == 16 && !SRC && NB == 2 ? 3 : 2)))) k_fused(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxes,
                                                      Closures c, double co0, double co1, double co2, StageArgs sa,
                                                      WrapArgs wa, Cover cov, UncovSrc us, NbMap nbm,
@@ -245,7 +249,7 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
   const gdouble* s1base = gptr(S1.p) + S1.off;
   const int s1off = min(gi, xhi) + min(gj, yhi) * int(S1.js);
   double pre[C::NLOAD][5];
-  auto load_plane = [&](int p) {
+  auto load_plane = [&](int p, bool below = false) {
     if constexpr (NB == 1) {
       nb_refresh(p);
 #pragma unroll
@@ -264,20 +268,23 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
       const gdouble* pu = u0base + int64_t(p) * S.ks;
 #pragma unroll
       for (int s = 0; s < C::NLOAD; ++s) {
+        const int o = EDGE && below && p < cov.lo[2] - 2 ? max(loff[s], cov.below) : loff[s];
         if ((s_um[s * NT + tid] >> b) & 1u) {
 #pragma unroll
-          for (int n = 0; n < 5; ++n) pre[s][n] = pu[n * S.ns + loff[s]];
+          for (int n = 0; n < 5; ++n) pre[s][n] = pu[n * S.ns + o];
         } else {
 #pragma unroll
-          for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + loff[s]];
+          for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + o];
         }
       }
     } else {
       const gdouble* pb = sbase + int64_t(p) * S.ks;
 #pragma unroll
-      for (int s = 0; s < C::NLOAD; ++s)
+      for (int s = 0; s < C::NLOAD; ++s) {
+        const int o = EDGE && below && p < cov.lo[2] - 2 ? max(loff[s], cov.below) : loff[s];
 #pragma unroll
-        for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + loff[s]];
+        for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + o];
+      }
     }
   };
   // order 6: the own column's conserved state two planes above an
@@ -287,8 +294,9 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
     if (wa.on) p = p < wa.lo[2] ? p + wa.len[2] : (p >= wa.lo[2] + wa.len[2] ? p - wa.len[2] : p);
     const bool from_u0 = UCS && ((um_own >> (((p - us.lo[2]) >> us.sh) - zb0)) & 1u);
     const gdouble* pb = (from_u0 ? u0base : sbase) + int64_t(p) * S.ks;
+    const int o = EDGE && p > cov.hi[2] + 2 ? min(soff, cov.above) : soff;
 #pragma unroll
-    for (int n = 0; n < 5; ++n) o2n[n] = pb[n * S.ns + soff];
+    for (int n = 0; n < 5; ++n) o2n[n] = pb[n * S.ns + o];
   };
   auto store_plane = [&](int p) {
     double* sq = s_q[p & 1];
@@ -322,7 +330,7 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
   for (int n = 0; n < 4; ++n) rm1[n] = 0.0;
 
   // prologue: plane kfirst into LDS
-  load_plane(kfirst);
+  load_plane(kfirst, true);
   store_plane(kfirst);
   load_plane(kfirst + 1);
   if (H == 3) load_own(kfirst + 2);
@@ -620,8 +628,8 @@ __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(H =
   }
 }
 
-#define AMR_FUSED_LAUNCH(UCS_, SRC_, NB_)                                                                     \
-  hipLaunchKernelGGL((k_fused<H, VISC, TX, TY, UCS_, SRC_, NB_>), dim3(ntiles), dim3(TX * TY), 0, st, tiles, \
+#define AMR_FUSED_LAUNCH(UCS_, SRC_, NB_, EDGE_)                                                                     \
+  hipLaunchKernelGGL((k_fused<H, VISC, TX, TY, UCS_, SRC_, NB_, EDGE_>), dim3(ntiles), dim3(TX * TY), 0, st, tiles, \
                      boxes, c, co[0], co[1], co[2], sa, wa, cov, us, nbm, s1, sin, out)
 
 template <int H, bool VISC, int TX, int TY>
@@ -632,21 +640,33 @@ void launch_t(const TileDev* tiles, int ntiles, const BoxDev* boxes, const Closu
   if constexpr (H <= 2) {
     if (nbm.on) {
       if (nbm.ustride) {
-        if (src) AMR_FUSED_LAUNCH(false, true, 2);
-        else AMR_FUSED_LAUNCH(false, false, 2);
+        if (src) AMR_FUSED_LAUNCH(false, true, 2, false);
+        else AMR_FUSED_LAUNCH(false, false, 2, false);
       } else {
-        if (src) AMR_FUSED_LAUNCH(false, true, 1);
-        else AMR_FUSED_LAUNCH(false, false, 1);
+        if (src) AMR_FUSED_LAUNCH(false, true, 1, false);
+        else AMR_FUSED_LAUNCH(false, false, 1, false);
+      }
+      return;
+    }
+  }
+  if constexpr (H == 3) {
+    if (cov.edge) {
+      if (us.on) {
+        if (src) AMR_FUSED_LAUNCH(true, true, 0, true);
+        else AMR_FUSED_LAUNCH(true, false, 0, true);
+      } else {
+        if (src) AMR_FUSED_LAUNCH(false, true, 0, true);
+        else AMR_FUSED_LAUNCH(false, false, 0, true);
       }
       return;
     }
   }
   if (us.on) {
-    if (src) AMR_FUSED_LAUNCH(true, true, 0);
-    else AMR_FUSED_LAUNCH(true, false, 0);
+    if (src) AMR_FUSED_LAUNCH(true, true, 0, false);
+    else AMR_FUSED_LAUNCH(true, false, 0, false);
   } else {
-    if (src) AMR_FUSED_LAUNCH(false, true, 0);
-    else AMR_FUSED_LAUNCH(false, false, 0);
+    if (src) AMR_FUSED_LAUNCH(false, true, 0, false);
+    else AMR_FUSED_LAUNCH(false, false, 0, false);
   }
 }
 #undef AMR_FUSED_LAUNCH

@@ -181,16 +181,20 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
     }
   }
   double pre[2][5];
-  auto load = [&](int s, int p) {
+  // `below`, `above`: may be a plane that the array holds in part (Cover)
+  auto load = [&](int s, int p, bool below = false, bool above = false) {
     if (wa.on) p = p < wa.lo[2] ? p + wa.len[2] : (p >= wa.lo[2] + wa.len[2] ? p - wa.len[2] : p);
     const gdouble* pb = sbase + int64_t(p) * S.ks;
+    int o = loff[s];
+    if (LEVEL && below && p < cov.lo[2] - 2) o = max(o, cov.below);
+    if (LEVEL && above && p > cov.hi[2] + 2) o = min(o, cov.above);
     if (UCS && ((s_um[s * NT + tid] >> (((p - us.lo[2]) >> us.sh) - zb0)) & 1u)) {
       const gdouble* pu = u0base + int64_t(p) * S.ks;
 #pragma unroll
-      for (int n = 0; n < 5; ++n) pre[s][n] = pu[n * S.ns + loff[s]];
+      for (int n = 0; n < 5; ++n) pre[s][n] = pu[n * S.ns + o];
     } else {
 #pragma unroll
-      for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + loff[s]];
+      for (int n = 0; n < 5; ++n) pre[s][n] = pb[n * S.ns + o];
     }
   };
   // the finished plane's own conserved state and s1, clamped into the valid
@@ -224,7 +228,7 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
       for (int n = 0; n < NPRIM; ++n) s_q[n * PL + hcell] = hn[n];
   };
 
-  load(0, k0 - 3);
+  load(0, k0 - 3, true);
   convert(0, q3);
   load(0, k0 - 2);
   load(1, k0 - 2);
@@ -252,7 +256,7 @@ k_fused_keep6(const TileDev* __restrict__ tiles, const BoxDev* __restrict__ boxe
     const bool inner = p > k0 && p <= k0 + nz;  // x/y work on the plane in LDS, p - 1
     // ---- own column of plane p: its z pairs
     convert(0, q0);
-    if (p < k0 + nz + 2) load(0, p + 1);
+    if (p < k0 + nz + 2) load(0, p + 1, false, true);
     {
       const Cell o{q0[QRHO], q0[QU], q0[QV], q0[QW], q0[QT], q0[QPRES]};
       double t[5];

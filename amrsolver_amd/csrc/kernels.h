@@ -108,13 +108,19 @@ struct WrapArgs {
 // instead of box by box, so they cross box boundaries.  [lo, hi] is the
 // bounding box of the boxes; bits (null when the bounding box is fully
 // covered) marks covered blocks of 2^sh cells a side, x fastest, nb blocks
-// per direction.  Only covered cells are written.
+// per direction.  Only covered cells are written.  below, above: order 6 loads
+// the planes lo[2] - 3 and hi[2] + 3 too, of which the array is known to hold
+// only what lies in a box's window: the lowest and the highest offset from those
+// planes that a load may have (a lane beyond takes that element; none of its
+// cells in reach of the plane is covered); edge: whether a lane can be.  U^n's
+// windows lie as the stage input's do.
 struct Cover {
   int on;
   int lo[3], hi[3];
   int nb[3];
   int sh;
   const unsigned* bits;
+  int below, above, edge;
 };
 
 // Owner map of a level for direct neighbour reads by the fused kernel's

@@ -68,7 +68,7 @@ def test_inviscid_order_2_with_neighbour_reads_keeps_three_waves(kernels):
     """Boxes with equal strides, KEEP order 2 without viscosity, 16x16 columns:
     at two waves (170 registers or more) 128x100x100 in 64x20x10 boxes takes
     224 us a step, at three 209."""
-    k = kernels["k_fused<1, false, 16, 16, false, false, 2>"]
+    k = kernels["k_fused<1, false, 16, 16, false, false, 2, false>"]
     assert _waves(k) >= 3 and k[".vgpr_spill_count"] == 0
 
 
