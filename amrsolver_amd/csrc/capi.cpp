@@ -3918,6 +3918,7 @@ int amr_adjoint_run(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme
     *sa = StageArgs{c2, nullptr, sch->order_rk, sch->stages_rk, s};
     return r;
   };
+  const bool fused = fused_path(bt, *sch, nullptr);
   // forward step n (global index) on stream sx; the last stage is skipped on
   // request
   auto run_step = [&](int n, bool skip_last, hipStream_t sx) -> int {
@@ -3925,7 +3926,8 @@ int amr_adjoint_run(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme
     for (int s = 0; s < nst; ++s) {
       DescSet* sin = R->sb(seg, nl, s);
       // stage inputs need their ghost cells (for the forward and the reverse
-      // sweep) unless the level is one periodic array read through images
+      // sweep) unless the level is one periodic array read through images, as
+      // every reverse kernel does and of the forward ones the fused
       const bool need_fill = !wrap_ok(bt, sin);
       if (skip_last && s == nst - 1) {
         // the stage itself is not needed, but the reverse sweep reads its
@@ -3945,7 +3947,7 @@ int amr_adjoint_run(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme
       else if (n + 1 == nsteps) out = R->uf();
       else if ((n + 1) % k == 0) out = R->ck(seg + 1);
       else out = R->sb(seg, nl + 1, 0);
-      if (need_fill && (r = enqueue_fill(bt, sin, false, sx))) return r;
+      if ((need_fill || !fused) && (r = enqueue_fill(bt, sin, false, sx))) return r;
       if ((r = do_stage(bt, *cls, *sch, sa, s1, sin, out, nullptr, sx))) return r;
     }
     return AMR_OK;
@@ -3966,7 +3968,7 @@ int amr_adjoint_run(amr_boxtab_t bt, const amr_closures_t* cls, const amr_scheme
   // (no box-table workspace) the recompute of segment seg-1 runs on a second
   // stream while segment seg is reversed: the forward kernel of a small level
   // leaves most CUs to the reverse kernels.
-  const bool overlap = R->nseg > 2 && fused_path(bt, *sch, nullptr);
+  const bool overlap = R->nseg > 2 && fused;
   hipStream_t sr = st;
   if (overlap) {
     if (!bt->aux) HIPCHK(hipStreamCreateWithFlags(&bt->aux, hipStreamNonBlocking));
